@@ -375,17 +375,11 @@ int dev_upload(Tp** dst, const std::vector<Tp>& src, std::vector<void*>& owned, 
 
 }  // namespace
 
-hipError_t launch_int1e(const asuka_jk_ctx* ctx, double* S, double* T, double* V, hipStream_t s);
 hipError_t launch_eri_deriv(const DevBasis& b, const ClassWork& w, const double* D, const double* WJ,
                             const double* WK, const int* shell_atom, double* grad, hipStream_t s);
 hipError_t launch_eri_deriv_fast(const DevBasis& b, const ClassWork& w, const double* D, const double* WJ,
                                  const double* WK, const int* shell_atom, int natm, double* grad, hipStream_t s,
                                  bool* handled);
-hipError_t launch_int1e_grad(const DevBasis& b, const int* pstart, const int* pnum, const double* pexp,
-                             const double* pcoef, int natm, const double* axyz, const double* aZ,
-                             const int* shell_atom, const double* Dh, const double* Ws, double* grad,
-                             hipStream_t s);
-
 struct asuka_jk_ctx {
   int device = 0;
   int nshell = 0, nao = 0, nsp = 0, natm = 0, max_l = 0;
@@ -452,6 +446,8 @@ struct asuka_jk_ctx {
   int* d_prim_num = nullptr;
   double* d_prim_exp = nullptr;
   double* d_prim_coef = nullptr;
+  int* d_cls_sp = nullptr;  // shell pairs sorted by class (Int1eArgs)
+  int cls_off[(ASUKA_LMAX + 1) * (ASUKA_LMAX + 2) / 2 + 1] = {0};
   unsigned long long* d_counters = nullptr;
   unsigned int* d_queue = nullptr;  // one work-queue head per class pair
   hipEvent_t ev_start = nullptr, ev_stop = nullptr;
@@ -816,6 +812,16 @@ static int ctx_build(const asuka_basis_desc* bd, const std::vector<int>* shell_m
   if ((rc = dev_upload(&d_pp, ctx->pp, own, s))) return rc;
   if ((rc = dev_upload(&d_ppf, ctx->ppf, own, s))) return rc;
   if ((rc = dev_upload(&ctx->d_shell_atom, ctx->shell_atom, own, s))) return rc;
+  {  // shell pairs by class, in pair order within a class (one-electron kernels)
+    const int nc = pair_class(ASUKA_LMAX, ASUKA_LMAX) + 1;
+    auto cls = [&](int sp) { return pair_class(ctx->shell_l[ctx->sp_A[sp]], ctx->shell_l[ctx->sp_B[sp]]); };
+    std::vector<int> cnt(nc + 1, 0), list(ctx->nsp);
+    for (int sp = 0; sp < ctx->nsp; ++sp) ++cnt[cls(sp) + 1];
+    for (int c = 0; c < nc; ++c) cnt[c + 1] += cnt[c];
+    std::copy(cnt.begin(), cnt.end(), ctx->cls_off);
+    for (int sp = 0; sp < ctx->nsp; ++sp) list[cnt[cls(sp)]++] = sp;
+    if ((rc = dev_upload(&ctx->d_cls_sp, list, own, s))) return rc;
+  }
   {
     std::vector<int> ps(bd->shell_prim_start, bd->shell_prim_start + nshell), pn(bd->shell_nprim, bd->shell_nprim + nshell);
     std::vector<double> pe(bd->prim_exp, bd->prim_exp + bd->nprim), pc(bd->prim_coef, bd->prim_coef + bd->nprim);
@@ -1440,6 +1446,21 @@ static ClassWork work_of(const asuka_jk_ctx* ctx, const ClassPairHost& cp, int i
   w.queue32 = ctx->d_queue + std::max<size_t>(1, ctx->cps.size()) + index;
   w.wpg = cp.wpg;
   return w;
+}
+
+static Int1eArgs int1e_args(const asuka_jk_ctx* ctx) {
+  Int1eArgs g{};
+  g.pstart = ctx->d_prim_start;
+  g.pnum = ctx->d_prim_num;
+  g.pexp = ctx->d_prim_exp;
+  g.pcoef = ctx->d_prim_coef;
+  g.natm = ctx->natm;
+  g.axyz = ctx->d_atom_xyz;
+  g.aZ = ctx->d_atom_Z;
+  g.cls_sp = ctx->d_cls_sp;
+  std::copy(std::begin(ctx->cls_off), std::end(ctx->cls_off), g.cls_off);
+  g.shell_atom = ctx->d_shell_atom;
+  return g;
 }
 
 static inline unsigned grid_for(long long n, int block) {
@@ -2074,7 +2095,7 @@ int asuka_int1e(asuka_jk_ctx* ctx, double* S, double* T, double* V, void* stream
   if (!ctx) return fail(ASUKA_E_INVALID, "ctx must be non-null");
   if (reject_batch(ctx)) return ASUKA_E_INVALID;
   if (V && ctx->natm <= 0) return fail(ASUKA_E_INVALID, "V needs atoms (natm > 0)");
-  HIP_CHECK(launch_int1e(ctx, S, T, V, (hipStream_t)stream));
+  HIP_CHECK(launch_int1e(ctx->dev, int1e_args(ctx), S, T, V, (hipStream_t)stream));
   return ASUKA_OK;
 }
 
@@ -2112,8 +2133,9 @@ int asuka_int1e_grad(asuka_jk_ctx* ctx, const double* Dh, const double* Ws, doub
   hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, s, grad, (long long)3 * ctx->natm, 0.0);
   HIP_CHECK(hipGetLastError());
   if (!Dh && !Ws) return ASUKA_OK;
-  HIP_CHECK(launch_int1e_grad(ctx->dev, ctx->d_prim_start, ctx->d_prim_num, ctx->d_prim_exp, ctx->d_prim_coef,
-                              ctx->natm, ctx->d_atom_xyz, ctx->d_atom_Z, ctx->d_shell_atom, Dh, Ws, grad, s));
+  Int1eArgs g = int1e_args(ctx);
+  g.grad = grad;
+  HIP_CHECK(launch_int1e_grad(ctx->dev, g, Dh, Ws, s));
   return ASUKA_OK;
 }
 
@@ -2136,150 +2158,3 @@ int asuka_rys_roots_device(int n, int64_t npts, const double* T, double* x, doub
 }
 
 }  // extern "C"
-
-// ---------------------------------------------------------------------------
-// One-electron integrals, one thread per shell pair.
-// S and T: 1-D overlap recursion and the kinetic-from-overlap relation
-// (asuka/integrals/int1e_cart.py:77-115, :758-787). V: Rys quadrature with a
-// point-charge ket (the q -> infinity limit of the ERI recursion):
-// G[a+1] = (PA - x PC) G[a] + a (1-x)/(2p) G[a-1], HRR on the bra, weight
-// -Z 2 pi / p exp(-mu AB^2) sum_u w_u Ix Iy Iz, T = p |PC|^2; equal to the
-// reference's McMurchie-Davidson form (int1e_cart.py:1031-1190).
-// ---------------------------------------------------------------------------
-namespace {
-
-constexpr int L1 = ASUKA_LMAX;
-constexpr int LT = L1 + 3;  // overlap table needs lb + 2
-
-__device__ void overlap_1d(int la, int lb, double a, double b, double A, double B, double S[L1 + 1][LT]) {
-  const double p = a + b, ip = 1.0 / p, mu = a * b * ip;
-  const double Px = (a * A + b * B) * ip, PA = Px - A, PB = Px - B, AB = A - B;
-  for (int i = 0; i <= L1; ++i)
-    for (int j = 0; j < LT; ++j) S[i][j] = 0.0;
-  S[0][0] = sqrt(3.14159265358979323846 * ip) * exp(-mu * AB * AB);
-  const double i2p = 0.5 * ip;
-  for (int j = 0; j < lb; ++j) S[0][j + 1] = PB * S[0][j] + (j > 0 ? j * i2p * S[0][j - 1] : 0.0);
-  for (int i = 0; i < la; ++i) {
-    S[i + 1][0] = PA * S[i][0] + (i > 0 ? i * i2p * S[i - 1][0] : 0.0);
-    for (int j = 0; j < lb; ++j)
-      S[i + 1][j + 1] = PA * S[i][j + 1] + (i > 0 ? i * i2p * S[i - 1][j + 1] : 0.0) + (j + 1) * i2p * S[i][j];
-  }
-}
-
-__device__ double kin1d(double S[L1 + 1][LT], int i, int j, double b) {
-  double v = b * (2.0 * j + 1.0) * S[i][j] - 2.0 * b * b * S[i][j + 2];
-  if (j >= 2) v -= 0.5 * (double)(j * (j - 1)) * S[i][j - 2];
-  return v;
-}
-
-// 1-D nuclear-attraction factor for one root: I(i, j), i <= la, j <= lb.
-__device__ double nuc1d(int i, int j, double PA, double PC, double AB, double x, double i2p) {
-  double G[2 * L1 + 1];
-  const double c0 = PA - x * PC, b1 = (1.0 - x) * i2p;
-  G[0] = 1.0;
-  const int n = i + j;
-  if (n > 0) G[1] = c0;
-  for (int a = 1; a < n; ++a) G[a + 1] = c0 * G[a] + a * b1 * G[a - 1];
-  // (i, j) = sum_k C(j,k) AB^(j-k) G[i+k]
-  double out = 0.0, binom = 1.0;
-  for (int k = 0; k <= j; ++k) {
-    double pw = 1.0;
-    for (int e = 0; e < j - k; ++e) pw *= AB;
-    out += binom * pw * G[i + k];
-    binom = binom * (double)(j - k) / (double)(k + 1);
-  }
-  return out;
-}
-
-__global__ void k_int1e(const DevBasis b, const int* pstart, const int* pnum, const double* pexp, const double* pcoef,
-                        int natm, const double* axyz, const double* aZ, double* S, double* T, double* V) {
-  const int sp = blockIdx.x * blockDim.x + threadIdx.x;
-  if (sp >= b.nsp) return;
-  const int A = b.sp_A[sp], B = b.sp_B[sp];
-  const int la = b.shell_l[A], lb = b.shell_l[B];
-  const int nA = ncart_c(la), nB = ncart_c(lb);
-  int ax[10], ay[10], az[10], bx[10], by[10], bz[10];
-  {
-    int i = 0;
-    for (int x = la; x >= 0; --x)
-      for (int y = la - x; y >= 0; --y) {
-        ax[i] = x;
-        ay[i] = y;
-        az[i] = la - x - y;
-        ++i;
-      }
-    i = 0;
-    for (int x = lb; x >= 0; --x)
-      for (int y = lb - x; y >= 0; --y) {
-        bx[i] = x;
-        by[i] = y;
-        bz[i] = lb - x - y;
-        ++i;
-      }
-  }
-  double s[100], t[100], v[100];
-  for (int i = 0; i < nA * nB; ++i) s[i] = t[i] = v[i] = 0.0;
-  const double* cA = b.shell_xyz + 3 * A;
-  const double* cB = b.shell_xyz + 3 * B;
-  const double ABx = cA[0] - cB[0], ABy = cA[1] - cB[1], ABz = cA[2] - cB[2];
-  const double AB2 = ABx * ABx + ABy * ABy + ABz * ABz;
-  const int nr = (la + lb) / 2 + 1;
-  for (int ia_p = 0; ia_p < pnum[A]; ++ia_p)
-    for (int ib_p = 0; ib_p < pnum[B]; ++ib_p) {
-      const double a = pexp[pstart[A] + ia_p], bb = pexp[pstart[B] + ib_p];
-      const double c = pcoef[pstart[A] + ia_p] * pcoef[pstart[B] + ib_p];
-      if (c == 0.0) continue;
-      double Sx[L1 + 1][LT], Sy[L1 + 1][LT], Sz[L1 + 1][LT];
-      overlap_1d(la, lb + 2, a, bb, cA[0], cB[0], Sx);
-      overlap_1d(la, lb + 2, a, bb, cA[1], cB[1], Sy);
-      overlap_1d(la, lb + 2, a, bb, cA[2], cB[2], Sz);
-      for (int i = 0; i < nA; ++i)
-        for (int j = 0; j < nB; ++j) {
-          const double sx = Sx[ax[i]][bx[j]], sy = Sy[ay[i]][by[j]], sz = Sz[az[i]][bz[j]];
-          s[i * nB + j] += c * sx * sy * sz;
-          t[i * nB + j] += c * (kin1d(Sx, ax[i], bx[j], bb) * sy * sz + sx * kin1d(Sy, ay[i], by[j], bb) * sz +
-                                sx * sy * kin1d(Sz, az[i], bz[j], bb));
-        }
-      if (!V) continue;
-      const double p = a + bb, ip = 1.0 / p;
-      const double Px = (a * cA[0] + bb * cB[0]) * ip, Py = (a * cA[1] + bb * cB[1]) * ip,
-                   Pz = (a * cA[2] + bb * cB[2]) * ip;
-      const double Kab = exp(-a * bb * ip * AB2);
-      for (int ic = 0; ic < natm; ++ic) {
-        const double Z = aZ[ic];
-        if (Z == 0.0) continue;
-        const double PCx = Px - axyz[3 * ic], PCy = Py - axyz[3 * ic + 1], PCz = Pz - axyz[3 * ic + 2];
-        const double Targ = p * (PCx * PCx + PCy * PCy + PCz * PCz);
-        const double pref = -Z * 2.0 * 3.14159265358979323846 * ip * Kab * c;
-        for (int u = 0; u < nr; ++u) {
-          double xr, wr;
-          rys_root_dev(nr, u, Targ, xr, wr);
-          for (int i = 0; i < nA; ++i)
-            for (int j = 0; j < nB; ++j) {
-              const double Ix = nuc1d(ax[i], bx[j], Px - cA[0], PCx, ABx, xr, 0.5 * ip);
-              const double Iy = nuc1d(ay[i], by[j], Py - cA[1], PCy, ABy, xr, 0.5 * ip);
-              const double Iz = nuc1d(az[i], bz[j], Pz - cA[2], PCz, ABz, xr, 0.5 * ip);
-              v[i * nB + j] += pref * wr * Ix * Iy * Iz;
-            }
-        }
-      }
-    }
-  const long long N = b.nao;
-  const int a0 = b.shell_ao[A], b0 = b.shell_ao[B];
-  for (int i = 0; i < nA; ++i)
-    for (int j = 0; j < nB; ++j) {
-      const long long r = a0 + i, cc = b0 + j;
-      if (S) S[r * N + cc] = S[cc * N + r] = s[i * nB + j];
-      if (T) T[r * N + cc] = T[cc * N + r] = t[i * nB + j];
-      if (V) V[r * N + cc] = V[cc * N + r] = v[i * nB + j];
-    }
-}
-
-}  // namespace
-
-hipError_t launch_int1e(const asuka_jk_ctx* ctx, double* S, double* T, double* V, hipStream_t s) {
-  hipLaunchKernelGGL(k_int1e, dim3((ctx->nsp + 63) / 64), dim3(64), 0, s, ctx->dev, ctx->d_prim_start,
-                     ctx->d_prim_num, ctx->d_prim_exp, ctx->d_prim_coef, ctx->natm, ctx->d_atom_xyz, ctx->d_atom_Z, S,
-                     T, V);
-  return hipGetLastError();
-}

@@ -341,6 +341,26 @@ __device__ inline bool decode_work(const ClassWork& w, long long k, int& P, int&
   return true;
 }
 
+// Inputs of the one-electron kernels (int1e.hip): the basis' primitives, the
+// nuclei, the shell pairs sorted by class (la (la + 1) / 2 + lb) and, for the
+// gradient, the shells' atoms and the output.
+struct Int1eArgs {
+  const int* pstart;
+  const int* pnum;
+  const double* pexp;
+  const double* pcoef;
+  int natm;
+  const double* axyz;
+  const double* aZ;
+  const int* cls_sp;
+  int cls_off[(ASUKA_LMAX + 1) * (ASUKA_LMAX + 2) / 2 + 1];
+  const int* shell_atom;
+  double* grad;  // (natm, 3)
+  int lg_group;  // log2 of the lanes over nuclei (set by the launcher)
+};
+hipError_t launch_int1e(const DevBasis& b, Int1eArgs g, double* S, double* T, double* V, hipStream_t s);
+hipError_t launch_int1e_grad(const DevBasis& b, Int1eArgs g, const double* Dh, const double* Ws, hipStream_t s);
+
 // Launchers (defined in jk_generic.hip / jk_fast.hip).
 hipError_t launch_eri_generic(const DevBasis& b, const ClassWork& w, const EriOut& o, hipStream_t s);
 // Wave-cooperative class templates (jk_coop.hip); *handled is false for classes it does not serve.
