@@ -107,13 +107,82 @@ struct ClassPairHost {
   long long rtask_off = 0;                // first of its remapped row tasks (routed mixed builds)
 };
 
+// Slices of wave units (WaveUnit). A lane runs the primitive quartets of its
+// shell quartet one after another, so a class pair with few units takes as
+// long as its longest unit: one water cc-pVDZ, (00|00), 1.7 ms for 45 x 45
+// primitive quartets on 560 waves. Units of the register kernels longer than
+// 1 / kSliceWaves of the class pair's work are therefore cut into blocks of
+// bra and ket primitive pairs, down to a size at which the transfer and
+// digestion that every slice repeats stay a small share: slice_min primitive
+// quartets, fewer for more roots (a primitive quartet of a class with n roots
+// costs about n^2 times as much; 24, 96 and 192 / n^2 were measured 9 % faster,
+// 32 % and 65 % slower than 48 for one water, and 2 %, 3 % and 4 % slower for
+// (H2O)7). Large contexts have no such unit and are left alone. Measured with
+// kFillTasks: one water cc-pVDZ, mixed Fock build 2.37 -> 0.60 ms, (H2O)7 FP64
+// 4.66 -> 3.46 ms, (H2O)2 cc-pVTZ J/K 8.7 -> 3.8 ms, (H2O)5 two densities 3.68
+// -> 2.41 ms.
+static constexpr long long kSliceWaves = 8192;
+static inline long long slice_min(int nroots) { return std::max(2, 48 / (nroots * nroots)); }
+
+// blk_k: largest primitive-pair count of each 64-position ket block.
+static void slice_units(const std::vector<int>& blk_k, ClassPairHost& cp, std::vector<WaveUnit>& units) {
+  const int nit = eri_fast_nch(cp.la, cp.lb, cp.lc, cp.ld);
+  if (nit <= 0 || cp.rows.empty()) return;
+  const size_t u0 = (size_t)cp.unit_start;
+  auto work = [&](const WaveUnit& u) { return (long long)u.i1 * blk_k[(size_t)u.col >> 6]; };  // primitive quartets
+  long long total = 0, longest = 0;
+  for (size_t k = u0; k < units.size(); ++k) {
+    const long long w = work(units[k]);
+    total += w * nit;
+    longest = std::max(longest, w);
+  }
+  const long long most = std::max(slice_min((cp.la + cp.lb + cp.lc + cp.ld) / 2 + 1), total / kSliceWaves);
+  if (longest <= most) return;
+  std::vector<WaveUnit> out;
+  for (auto& row : cp.rows) {
+    const int first = (int)out.size();
+    for (int k = row.first; k < row.first + row.second; ++k) {
+      const WaveUnit u = units[u0 + k];
+      const int ni = (int)u.i1;
+      const long long w = work(u);
+      const int kcd = blk_k[(size_t)u.col >> 6];
+      if (w <= most || ni >= kUnitAll || kcd >= kUnitAll) {
+        out.push_back(u);
+        continue;
+      }
+      const long long n = (w + most - 1) / most;
+      const int si = (int)std::min<long long>(ni, n), sj = (int)std::min<long long>(kcd, (n + si - 1) / si);
+      for (int a = 0; a < si; ++a)
+        for (int c = 0; c < sj; ++c) {
+          WaveUnit v = u;
+          v.i0 = (unsigned)((long long)ni * a / si);
+          v.i1 = (unsigned)((long long)ni * (a + 1) / si);
+          v.tail = a == si - 1;
+          v.j0 = (unsigned)((long long)kcd * c / sj);
+          v.j1 = c == sj - 1 ? (unsigned)kUnitAll : (unsigned)((long long)kcd * (c + 1) / sj);
+          out.push_back(v);
+        }
+    }
+    row = {first, (int)out.size() - first};
+  }
+  units.resize(u0);
+  units.insert(units.end(), out.begin(), out.end());
+}
+
 // Row tasks of a class pair: each row's wave units cut into
 // ceil(nu / task_units) tasks of balanced size, longest (in primitive
 // quartets) first, since workgroups pull them from a queue in order and the
-// tail of the launch is then made of short tasks.
+// tail of the launch is then made of short tasks. A class pair with few units
+// is cut finer, into about kFillTasks tasks (two workgroups a CU) of at least
+// one wave item per wavefront, so that its units spread over the chip (1024
+// measured 1-4 % slower below 10 molecules: each task flushes its LDS sums).
+static constexpr long long kFillTasks = 512;
 static std::vector<RowTask> make_tasks(const ClassPairHost& cp, const WaveUnit* units, const std::vector<int>& col,
                                        const std::vector<int>& pp_count, int task_units) {
   std::vector<RowTask> tasks;
+  const int nit = std::max(1, eri_fast_nch(cp.la, cp.lb, cp.lc, cp.ld));
+  task_units = (int)std::min<long long>(
+      task_units, std::max<long long>((cp.wpg + nit - 1) / nit, (cp.nunits + kFillTasks - 1) / kFillTasks));
   for (const auto& r : cp.rows) {
     const int nu = r.second;
     const int ntk = (nu + task_units - 1) / task_units;
@@ -122,12 +191,14 @@ static std::vector<RowTask> make_tasks(const ClassPairHost& cp, const WaveUnit* 
       tasks.push_back(RowTask{r.first + b0, b1 - b0});
     }
   }
+  auto cost = [&](const RowTask& t, const WaveUnit& u) {
+    const int j1 = std::min(pp_count[col[u.col]], (int)u.j1);
+    return (long long)t.nu * (u.i1 == kUnitAll ? pp_count[u.P] : (int)u.i1 - (int)u.i0) * (j1 - (int)u.j0);
+  };
   std::stable_sort(tasks.begin(), tasks.end(), [&](const RowTask& x, const RowTask& y) {
     const WaveUnit& ux = units[x.u0];
     const WaveUnit& uy = units[y.u0];
-    const long long cx = (long long)x.nu * pp_count[ux.P] * pp_count[col[ux.col]];
-    const long long cy = (long long)y.nu * pp_count[uy.P] * pp_count[col[uy.col]];
-    return cx > cy;
+    return cost(x, ux) > cost(y, uy);
   });
   return tasks;
 }
@@ -1160,6 +1231,9 @@ static int ctx_build(const asuka_basis_desc* bd, const std::vector<int>* shell_m
       groups[c].push_back(std::move(g));
     }
   }
+  std::vector<int> blk_k((col_all.size() + 63) / 64, 0);
+  for (size_t t = 0; t < col_all.size(); ++t)
+    if (col_all[t] >= 0) blk_k[t >> 6] = std::max(blk_k[t >> 6], ctx->pp_count[col_all[t]]);
   const double eps = ctx->eps_schwarz;
   for (int X = 0; X < ncls; ++X) {
     for (int Y = 0; Y <= X; ++Y) {
@@ -1241,7 +1315,14 @@ static int ctx_build(const asuka_basis_desc* bd, const std::vector<int>* shell_m
                   while (k < nabu && ctx->ppf[ctx->pp_start[P] + k].q >= thr) ++k;
                   nabu = k;
                 }
-                units.push_back(WaveUnit{P, kg.col_start + (int)c0, nc, nabu});
+                WaveUnit wu{};
+                wu.P = P;
+                wu.col = kg.col_start + (int)c0;
+                wu.ncol = (unsigned)nc;
+                wu.tail = 1;
+                wu.i1 = (unsigned)std::min(nabu, kUnitAll);
+                wu.j1 = kUnitAll;
+                units.push_back(wu);
               }
             }
           }
@@ -1269,6 +1350,7 @@ static int ctx_build(const asuka_basis_desc* bd, const std::vector<int>* shell_m
         }
       }
       cp.nseg = (int)segs.size() - cp.seg_start;
+      slice_units(blk_k, cp, units);
       cp.nunits = (long long)units.size() - cp.unit_start;
       {
         const std::vector<RowTask> tk = make_tasks(cp, units.data() + cp.unit_start, col_all, ctx->pp_count, task_units);

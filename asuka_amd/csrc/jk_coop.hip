@@ -119,7 +119,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4))) void
   for (long long k = blockIdx.x; k < w.nunits * 64; k += gridDim.x) {
     const WaveUnit un = w.units[k >> 6];
     const int jk = (int)(k & 63);
-    if (jk >= un.ncol) continue;  // uniform: one quartet per wave
+    if (jk >= (int)un.ncol) continue;  // uniform: one quartet per wave (units of these classes are never sliced)
     const int P = un.P;
     const int A = b.sp_A[P], B = b.sp_B[P];
     const double* cA = b.shell_xyz + 3 * A;

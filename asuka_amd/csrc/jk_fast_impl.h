@@ -273,8 +273,8 @@ struct RowAcc {
 // or -1 for D[c,d] from D and J[c,d] atomics on J.
 
 template <class PL, int CH, typename CT, bool FX>
-__device__ __forceinline__ void run_chunk(const DevBasis& b, const EriOut& o, int P, int Qp, int pos, int nab,
-                                          bool active, const CT* __restrict__ tab, const RowAcc& acc, double* jcd,
+__device__ __forceinline__ void run_chunk(const DevBasis& b, const EriOut& o, int P, int Qp, int pos,
+                                          const UnitRange& ur, bool active, const CT* __restrict__ tab, const RowAcc& acc, double* jcd,
                                           long long jb) {
   using CK = Chunk<PL, CH>;
   constexpr int NEL = CK::NEL, NFL = CK::NFL, NR = PL::NR;
@@ -294,9 +294,9 @@ __device__ __forceinline__ void run_chunk(const DevBasis& b, const EriOut& o, in
   // the ket pair's data by its position (pos: contiguous across the lanes)
   const int A = uni(b.sp_A[P]), B = uni(b.sp_B[P]);
   const double Ax = b.shell_xyz[3 * A], Ay = b.shell_xyz[3 * A + 1], Az = b.shell_xyz[3 * A + 2];
-  const int ab0 = uni(b.pp_start[P]);
+  const int ab0 = uni(b.pp_start[P]) + ur.i0, nab = ur.ni;  // the unit's bra primitive pairs
   const int2 kpp = b.kpp[pos];
-  const int ncd = active ? kpp.y : 0;  // (kpp.x, the first pair in the pair table, is for host-side use)
+  const int ncd = active ? min(kpp.y, ur.j1) : 0;  // (kpp.x, the first pair in the pair table, is for host-side use)
   // the primitive pairs in the precision of CT (the FP32 path reads the float
   // copy: no conversions in the primitive loop but P - Q, formed in FP64)
   using PPT = typename std::conditional<sizeof(CT) == 4, PrimPairF32, PrimPairF>::type;
@@ -321,8 +321,8 @@ __device__ __forceinline__ void run_chunk(const DevBasis& b, const EriOut& o, in
   // pairs are contiguous): slots ks0 + 64 j
   const int ks0 = (int)b.kpoff[uni(pos >> 6)] * 64 + (pos & 63);
   PPT Yn;
-  if (ncd > 0) Yn = load_ket<PPT>(b, ks0);
-  for (int j = 0; j < ncd; ++j) {
+  if (ur.j0 < ncd) Yn = load_ket<PPT>(b, ks0 + 64 * ur.j0);
+  for (int j = ur.j0; j < ncd; ++j) {
     const PPT Y = Yn;
     if (Y.q < kcut) break;  // per lane: the rest of its ket pairs are smaller
     if (j + 1 < ncd) Yn = load_ket<PPT>(b, ks0 + 64 * (j + 1));  // next ket pair, in flight during this one
@@ -612,25 +612,25 @@ __device__ __forceinline__ void run_chunk(const DevBasis& b, const EriOut& o, in
 
 template <class PL, int CH, typename CT, bool FX>
 __device__ __forceinline__ void dispatch_chunk(int chunk, const DevBasis& b, const EriOut& o, int P, int Qp, int pos,
-                                               int nab, bool active, const CT* __restrict__ tab, const RowAcc& acc,
+                                               const UnitRange& ur, bool active, const CT* __restrict__ tab, const RowAcc& acc,
                                                long long jb) {
   if constexpr (CH < PL::NCH) {
     if (chunk == CH) {
-      run_chunk<PL, CH, CT, FX>(b, o, P, Qp, pos, nab, active, tab, acc, nullptr, jb);
+      run_chunk<PL, CH, CT, FX>(b, o, P, Qp, pos, ur, active, tab, acc, nullptr, jb);
       return;
     }
-    dispatch_chunk<PL, CH + 1, CT, FX>(chunk, b, o, P, Qp, pos, nab, active, tab, acc, jb);
+    dispatch_chunk<PL, CH + 1, CT, FX>(chunk, b, o, P, Qp, pos, ur, active, tab, acc, jb);
   }
 }
 
 // The A chunks CA.. of C chunk CC, in sequence, carrying J[c,d] in jcd.
 template <class PL, int CC, int CA, typename CT, bool FX>
-__device__ __forceinline__ void run_agroup(const DevBasis& b, const EriOut& o, int P, int Qp, int pos, int nab,
-                                           bool active, const CT* __restrict__ tab, const RowAcc& acc, double* jcd,
+__device__ __forceinline__ void run_agroup(const DevBasis& b, const EriOut& o, int P, int Qp, int pos,
+                                           const UnitRange& ur, bool active, const CT* __restrict__ tab, const RowAcc& acc, double* jcd,
                                            long long jb) {
   if constexpr (CA < PL::SPLIT_A) {
-    run_chunk<PL, CA * PL::SPLIT_C + CC, CT, FX>(b, o, P, Qp, pos, nab, active, tab, acc, jcd, jb);
-    run_agroup<PL, CC, CA + 1, CT, FX>(b, o, P, Qp, pos, nab, active, tab, acc, jcd, jb);
+    run_chunk<PL, CA * PL::SPLIT_C + CC, CT, FX>(b, o, P, Qp, pos, ur, active, tab, acc, jcd, jb);
+    run_agroup<PL, CC, CA + 1, CT, FX>(b, o, P, Qp, pos, ur, active, tab, acc, jcd, jb);
   }
 }
 
@@ -638,14 +638,14 @@ __device__ __forceinline__ void run_agroup(const DevBasis& b, const EriOut& o, i
 // with the J[c,d] sums carried across the A chunks in registers, so J[c,d]
 // receives one atomic per element and quartet instead of one per A chunk.
 template <class PL, int CC, typename CT, bool FX>
-__device__ __forceinline__ void run_citem(const DevBasis& b, const EriOut& o, int P, int Qp, int pos, int nab,
-                                          bool active, const CT* __restrict__ tab, const RowAcc& acc, long long jb) {
+__device__ __forceinline__ void run_citem(const DevBasis& b, const EriOut& o, int P, int Qp, int pos,
+                                          const UnitRange& ur, bool active, const CT* __restrict__ tab, const RowAcc& acc, long long jb) {
   using CK = Chunk<PL, CC>;  // A chunk 0: the C range of every A chunk of CC
   constexpr int ND = PL::ND, NCDL = (CK::c1 - CK::c0) * ND;
   double jcd[NCDL];
 #pragma unroll
   for (int c = 0; c < NCDL; ++c) jcd[c] = 0.0;
-  run_agroup<PL, CC, 0, CT, FX>(b, o, P, Qp, pos, nab, active, tab, acc, jcd, jb);
+  run_agroup<PL, CC, 0, CT, FX>(b, o, P, Qp, pos, ur, active, tab, acc, jcd, jb);
   double* Jo = (o.mode == MODE_FOCK) ? o.F : o.J;
   if (Jo && active && P != Qp && jb >= 0) {
     const int lane = threadIdx.x & 63;
@@ -666,16 +666,16 @@ __device__ __forceinline__ void run_citem(const DevBasis& b, const EriOut& o, in
 // one chunk otherwise.
 template <class PL, int CC, typename CT, bool FX>
 __device__ __forceinline__ void dispatch_citem(int cc, const DevBasis& b, const EriOut& o, int P, int Qp, int pos,
-                                               int nab, bool active, const CT* __restrict__ tab, const RowAcc& acc,
+                                               const UnitRange& ur, bool active, const CT* __restrict__ tab, const RowAcc& acc,
                                                long long jb) {
   if constexpr (!PL::CARRY) {
-    dispatch_chunk<PL, 0, CT, FX>(cc, b, o, P, Qp, pos, nab, active, tab, acc, jb);
+    dispatch_chunk<PL, 0, CT, FX>(cc, b, o, P, Qp, pos, ur, active, tab, acc, jb);
   } else if constexpr (CC < PL::SPLIT_C) {
     if (cc == CC) {
-      run_citem<PL, CC, CT, FX>(b, o, P, Qp, pos, nab, active, tab, acc, jb);
+      run_citem<PL, CC, CT, FX>(b, o, P, Qp, pos, ur, active, tab, acc, jb);
       return;
     }
-    dispatch_citem<PL, CC + 1, CT, FX>(cc, b, o, P, Qp, pos, nab, active, tab, acc, jb);
+    dispatch_citem<PL, CC + 1, CT, FX>(cc, b, o, P, Qp, pos, ur, active, tab, acc, jb);
   }
 }
 
@@ -796,7 +796,7 @@ __global__ __launch_bounds__(kGroupThreads) void eri_fast_kernel(DevBasis b, Cla
       const int chunk = item / tk.nu;
       const int ui = item - chunk * tk.nu;
       const WaveUnit un = w.units[tk.u0 + ui];
-      bool active = lane < un.ncol;
+      bool active = lane < (int)un.ncol;
       // the lane's ket position: units start at 64-position block boundaries,
       // so every lane's position (tail lanes: padding) is inside the lists
       const int pos = un.col + lane;
@@ -812,29 +812,33 @@ __global__ __launch_bounds__(kGroupThreads) void eri_fast_kernel(DevBasis b, Cla
         if (lowp != kF32) continue;  // the other precision's kernel takes this unit
       }
       worked = true;
+      // the unit's primitive pairs (see run_chunk)
+      UnitRange ur = unit_range(un, b.pp_count[P], false);
+      ur.i0 = uni(ur.i0), ur.ni = uni(ur.ni), ur.j0 = uni(ur.j0), ur.j1 = uni(ur.j1);
       if (o.counters && chunk == 0) {
-        // statistics: one atomic per counter and wave
+        // statistics: one atomic per counter and wave; quartets are counted by
+        // their first slice
+        const bool first_slice = ur.i0 == 0 && ur.j0 == 0;
         const int A = b.sp_A[P], B = b.sp_B[P], C = b.sp_A[Qp], Dsh = b.sp_B[Qp];
         unsigned long long* cnt = o.counters + kCountStride * w.cp_index;
         const unsigned long long kq =
-            active ? (unsigned long long)b.pp_count0[P] * (unsigned long long)b.pp_count0[Qp] : 0ull;
+            active && first_slice ? (unsigned long long)b.pp_count0[P] * (unsigned long long)b.pp_count0[Qp] : 0ull;
         const int bin = (((A != B) << 2) | ((C != Dsh) << 1) | (P != Qp));
         for (int k = 0; k < 8; ++k) {
-          const unsigned long long m = __ballot(active && bin == k);
+          const unsigned long long m = __ballot(active && first_slice && bin == k);
           if (m && lane == 0) atomicAdd(cnt + k, (unsigned long long)__popcll(m));
         }
         const unsigned long long ksum = (unsigned long long)wave_sum((double)kq);
-        const unsigned long long nact = (unsigned long long)__popcll(__ballot(active));
+        const unsigned long long nact = (unsigned long long)__popcll(__ballot(active && first_slice));
         // primitive quartets the loops evaluate (after the primitive-quartet
         // cut) and the lane slots the wave spends on them (64 x the longest lane)
-        const int nabc = uni(o.eps_prim > 0.0 ? un.nab : b.pp_count[P]);
         long long nev = 0;
-        if (active && nabc > 0) {
-          const int cd0 = b.pp_start[Qp], ncd = b.pp_count[Qp];
-          const double kcut = o.eps_prim > 0.0 ? o.eps_prim / b.ppf[b.pp_start[P]].q : 0.0;
-          int j = 0;
+        if (active && ur.ni > 0) {
+          const int cd0 = b.pp_start[Qp], ncd = min(b.pp_count[Qp], ur.j1);
+          const double kcut = o.eps_prim > 0.0 ? o.eps_prim / b.ppf[b.pp_start[P] + ur.i0].q : 0.0;
+          int j = ur.j0;
           while (j < ncd && !(b.ppf[cd0 + j].q < kcut)) ++j;
-          nev = (long long)nabc * j;
+          nev = (long long)ur.ni * (j - ur.j0);
         }
         const double nevs = wave_sum((double)nev);
         double nmax = (double)nev;
@@ -852,11 +856,9 @@ __global__ __launch_bounds__(kGroupThreads) void eri_fast_kernel(DevBasis b, Cla
       }
       // inactive lanes (tail, screened) run with an empty primitive loop and no
       // atomics so the wave stays converged for the cross-lane reductions
-      // bra primitive pairs this unit evaluates (see run_chunk)
-      const int nab = uni(o.eps_prim > 0.0 ? un.nab : b.pp_count[P]);
       // the unit's block of the ket-position buffers (units start at block boundaries)
       const long long jb = o.jblk ? o.jblk[un.col >> 6] : -1LL;
-      dispatch_citem<PL, 0, CT, FX>(chunk, b, o, P, Qp, pos, nab, active, tab, acc, jb);
+      dispatch_citem<PL, 0, CT, FX>(chunk, b, o, P, Qp, pos, ur, active, tab, acc, jb);
     }
     if (use_acc) {
       if (worked && lane == 0) s_work = 1;

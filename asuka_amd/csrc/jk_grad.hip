@@ -108,7 +108,7 @@ __global__ __launch_bounds__(kWave) void eri_deriv_kernel(DevBasis b, ClassWork 
   // item k: ket k % 64 of wave unit k / 64 (one quartet per wave at a time)
   for (long long k = blockIdx.x; k < w.nunits * 64; k += gridDim.x) {
     const WaveUnit un = w.units[k >> 6];
-    if ((int)(k & 63) >= un.ncol) continue;  // uniform across the wave
+    if ((int)(k & 63) >= (int)un.ncol) continue;  // uniform across the wave
     const int P = un.P, Qp = w.col_pair[un.col + (int)(k & 63)];
     const int A = b.sp_A[P], B = b.sp_B[P], C = b.sp_A[Qp], Dsh = b.sp_B[Qp];
     const double* cA = b.shell_xyz + 3 * A;
@@ -121,8 +121,9 @@ __global__ __launch_bounds__(kWave) void eri_deriv_kernel(DevBasis b, ClassWork 
     const bool ab_neq = A != B, cd_neq = C != Dsh, bk = P != Qp;
     const double fj = (ab_neq ? 2.0 : 1.0) * (cd_neq ? 2.0 : 1.0);
     const double fk = bk ? 2.0 : 1.0;
-    const int ab0 = b.pp_start[P], nab = b.pp_count[P];
-    const int cd0 = b.pp_start[Qp], ncd = b.pp_count[Qp];
+    const UnitRange ur = unit_range(un, b.pp_count[P], true);  // the unit's primitive pairs
+    const int ab0 = b.pp_start[P] + ur.i0, nab = ur.ni;
+    const int cd0 = b.pp_start[Qp], ncd = min(b.pp_count[Qp], ur.j1);
 
     double gA[3] = {0, 0, 0}, gB[3] = {0, 0, 0}, gC[3] = {0, 0, 0};
     for (int c0 = 0; c0 < ncomp; c0 += kChunk) {
@@ -157,7 +158,7 @@ __global__ __launch_bounds__(kWave) void eri_deriv_kernel(DevBasis b, ClassWork 
 
       for (int i = 0; i < nab; ++i) {
         const PrimPair X = b.pp[ab0 + i];
-        for (int j = 0; j < ncd; ++j) {
+        for (int j = ur.j0; j < ncd; ++j) {
           const PrimPair Y = b.pp[cd0 + j];
           const double p = X.eta, q = Y.eta, alpha2 = 2.0 * X.a_exp, beta2 = 2.0 * X.b_exp, gamma2 = 2.0 * Y.a_exp;
           const double inv_pq = 1.0 / (p + q);

@@ -145,7 +145,7 @@ struct GradFastArgs {
 // lane's ket position (contiguous across the lanes; DevBasis::kpoff).
 template <int LA, int LB, int LC, int LD, int C0, int C1>
 __device__ __forceinline__ void deriv_unit(const DevBasis& b, const GradFastArgs& g, const double* tab, int P, int Qp,
-                                           int pos, bool active, double* sgrad, bool lds_grad) {
+                                           int pos, const UnitRange& ur, bool active, double* sgrad, bool lds_grad) {
   using DP = DPlan<LA, LB, LC, LD>;
   constexpr int NB = DP::NB, NC = DP::NC, ND = DP::ND;
   constexpr int NR = DP::NR, NM = DP::NMAX, MM = DP::MMAX;
@@ -191,8 +191,8 @@ __device__ __forceinline__ void deriv_unit(const DevBasis& b, const GradFastArgs
     bar[ci - C0] = v;
   }
   double gA[3] = {0, 0, 0}, gB[3] = {0, 0, 0}, gC[3] = {0, 0, 0};
-  const int ab0 = uni_g(b.pp_start[P]), nab = uni_g(b.pp_count[P]);
-  const int ncd = active ? b.kpp[pos].y : 0;
+  const int ab0 = uni_g(b.pp_start[P]) + ur.i0, nab = ur.ni;  // the unit's bra primitive pairs
+  const int ncd = active ? min(b.kpp[pos].y, ur.j1) : 0;
   // the lane's ket primitive pairs from the transposed tables (slots
   // ks0 + 64 j, field f at kp64[f * kslots + slot]): one contiguous load
   // per field across the wave (no prefetch of the next pair: its registers
@@ -212,7 +212,7 @@ __device__ __forceinline__ void deriv_unit(const DevBasis& b, const GradFastArgs
     y[8] = (kt + 8 * ns)[t];
     y[9] = (kt + 10 * ns)[t]; // exponent of the C primitive
   };
-  for (int j = 0; j < ncd; ++j) {
+  for (int j = ur.j0; j < ncd; ++j) {
     double y[10];
     ket(ks0 + 64 * j, y);
     const double q = y[0], iq = y[1], ckq = y[2], c2 = 2.0 * y[9];
@@ -291,15 +291,16 @@ __device__ __forceinline__ void deriv_unit(const DevBasis& b, const GradFastArgs
 
 template <int LA, int LB, int LC, int LD, int NCH, int CH>
 __device__ __forceinline__ void deriv_dispatch(int chunk, const DevBasis& b, const GradFastArgs& g, const double* tab,
-                                               int P, int Qp, int pos, bool active, double* sgrad, bool lds_grad) {
+                                               int P, int Qp, int pos, const UnitRange& ur, bool active, double* sgrad,
+                                               bool lds_grad) {
   if constexpr (CH < NCH) {
     constexpr int NCOMP = DPlan<LA, LB, LC, LD>::NCOMP;
     if (chunk == CH) {
-      deriv_unit<LA, LB, LC, LD, CH * NCOMP / NCH, (CH + 1) * NCOMP / NCH>(b, g, tab, P, Qp, pos, active, sgrad,
-                                                                            lds_grad);
+      deriv_unit<LA, LB, LC, LD, CH * NCOMP / NCH, (CH + 1) * NCOMP / NCH>(b, g, tab, P, Qp, pos, ur, active,
+                                                                            sgrad, lds_grad);
       return;
     }
-    deriv_dispatch<LA, LB, LC, LD, NCH, CH + 1>(chunk, b, g, tab, P, Qp, pos, active, sgrad, lds_grad);
+    deriv_dispatch<LA, LB, LC, LD, NCH, CH + 1>(chunk, b, g, tab, P, Qp, pos, ur, active, sgrad, lds_grad);
   }
 }
 
@@ -335,11 +336,13 @@ __global__ __launch_bounds__(kThreads) void eri_deriv_fast_kernel(DevBasis b, Cl
       const int chunk = item / tk.nu, ui = item - chunk * tk.nu;
       const WaveUnit un = w.units[tk.u0 + ui];
       const int P = uni_g(un.P);
-      const bool active = lane < un.ncol;
+      const bool active = lane < (int)un.ncol;
+      UnitRange ur = unit_range(un, b.pp_count[P], true);  // no primitive-quartet cut here
+      ur.i0 = uni_g(ur.i0), ur.ni = uni_g(ur.ni), ur.j0 = uni_g(ur.j0), ur.j1 = uni_g(ur.j1);
       const int Qp = w.col_pair[un.col + (active ? lane : 0)];
       // units start at 64-position blocks, so un.col + lane stays inside the
       // unit's block (padding positions for the inactive lanes)
-      deriv_dispatch<LA, LB, LC, LD, NCH, 0>(chunk, b, g, tab, P, Qp, un.col + lane, active, sgrad, lds_grad);
+      deriv_dispatch<LA, LB, LC, LD, NCH, 0>(chunk, b, g, tab, P, Qp, un.col + lane, ur, active, sgrad, lds_grad);
     }
     __syncthreads();  // s_task may be overwritten
   }

@@ -128,14 +128,25 @@ struct Segment {
 };
 
 // One wavefront's share of a segment: a bra pair and up to 64 consecutive
-// kets of its row (one per lane), so the bra side is uniform across the wave.
+// kets of its row (one per lane), so the bra side is uniform across the wave,
+// and of their primitive quartets the block of bra primitive pairs [i0, i1) and
+// ket primitive pairs [j0, j1): long primitive loops of small class pairs are
+// cut into several units (slices), whose contributions add up. i1 of the last
+// bra slice (tail) leaves out the bra pairs whose bound times the largest
+// ket-pair bound of the unit is below the primitive-quartet cut; kernels
+// without that cut (the derivatives) run it to the end.
+constexpr int kUnitAll = 16383;  // i1, j1: up to the last primitive pair
 struct WaveUnit {
-  int P;     // bra shell pair
-  int col;   // first ket, index into col_pair
-  int ncol;  // 1..64
-  int nab;   // bra primitive pairs to evaluate: those whose bound times the
-             // largest ket-pair bound of the unit reaches the primitive-quartet cut
+  int P;    // bra shell pair
+  int col;  // first ket, index into col_pair
+  unsigned long long ncol : 7;  // 1..64
+  unsigned long long tail : 1;
+  unsigned long long i0 : 14;
+  unsigned long long i1 : 14;
+  unsigned long long j0 : 14;
+  unsigned long long j1 : 14;
 };
+static_assert(sizeof(WaveUnit) == 16, "wave units are read as 16 bytes");
 
 // A workgroup's share: consecutive wave units [u0, u0 + nu) of one bra row.
 struct RowTask {
@@ -265,6 +276,20 @@ __device__ inline void mol_layout(const DevBasis& b, int A, long long& stride, l
 template <typename T>
 __device__ inline T* shifted(T* p, long long sh) {
   return p ? p + sh : p;
+}
+
+// The primitive pairs of a unit: bra pairs [i0, i0 + ni), ket pairs [j0, j1).
+struct UnitRange {
+  int i0, ni, j0, j1;
+};
+// nab: primitive pairs of the bra; full: without the primitive-quartet cut.
+__device__ __forceinline__ UnitRange unit_range(const WaveUnit& u, int nab, bool full) {
+  UnitRange r;
+  r.i0 = (int)u.i0;
+  r.ni = ((int)u.i1 == kUnitAll || (full && u.tail) ? nab : (int)u.i1) - r.i0;
+  r.j0 = (int)u.j0;
+  r.j1 = (int)u.j1 == kUnitAll ? 0x7fffffff : (int)u.j1;
+  return r;
 }
 
 __host__ __device__ constexpr inline int ncart_c(int l) { return (l + 1) * (l + 2) / 2; }
