@@ -90,6 +90,11 @@ SYMBOLS = [
     ("asuka_jk_build", ctypes.c_int, [_vp, _vp, _vp, _vp, ctypes.c_int, _vp]),
     ("asuka_jk_build_noalloc", ctypes.c_int, [_vp, _vp, _vp, _vp, ctypes.c_int, _vp]),
     ("asuka_scf_diis_solve", ctypes.c_int, [_vp, _vp, ctypes.c_int, _vp, _vp, _vp]),
+    ("asuka_scf_purify_max", ctypes.c_int, []),
+    ("asuka_scf_purify", ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_double, _vp, _vp, _vp,
+                                        _vp]),
+    ("asuka_scf_tc2_step", ctypes.c_int, [_vp, _vp, ctypes.c_int, ctypes.c_int, ctypes.c_double, _vp, _vp,
+                                          ctypes.c_int, _vp, _vp]),
     ("asuka_df_ctx_create", ctypes.c_int, [_vp, _vp, _vp, _vp]),
     ("asuka_df_ctx_destroy", ctypes.c_int, [_vp]),
     ("asuka_df_ctx_info", ctypes.c_int, [_vp, _vp]),

@@ -257,7 +257,7 @@ def rhf_direct(
         (the same projector, no eigensolver)."""
         if use_graph:
             Fo = X.T @ shifted(F) @ X
-            P, _ = _purify(torch, _sym(Fo), nocc, _purify_steps(torch, _sym(Fo), nocc) + 4)
+            P, _ = _purify_converged(torch, _sym(Fo), nocc)
             return None, None, _sym(2.0 * (X @ P @ X.T))
         e, Cm = _gen_eigh(torch, shifted(F), X)
         return e, Cm, _density(Cm, nocc)
@@ -351,6 +351,54 @@ def rhf_direct(
 _PURIFY_TOL = 1e-11  # ||P^2 - P||_F at which a purification stops updating
 
 
+def _purify_start(torch, Fo):
+    """(e1 - Fo)/(e1 - e0), [e0, e1] the Gershgorin interval of Fo: its spectrum in [0, 1], reversed."""
+    n = int(Fo.shape[0])
+    d = torch.diagonal(Fo)
+    r = Fo.abs().sum(dim=1) - d.abs()
+    e0 = (d - r).min()
+    e1 = (d + r).max()
+    return ((e1 * torch.eye(n, dtype=Fo.dtype, device=Fo.device) - Fo) / (e1 - e0)).contiguous()
+
+
+def _purify_run(torch, Fo, nocc: int, iters: int, chunk: int = 0):
+    """TC2 purification of the symmetric Fo in at most ``iters`` steps: (P, err,
+    step): err on the device; step() is the number of the step at which the
+    projector froze, 0 if it did not (a host read). Matrices up to asuka_scf_purify_max()
+    run in one kernel; larger ones take a product and asuka_scf_tc2_step per
+    step (with ``chunk`` the host looks every that many steps and stops early)."""
+    from .. import _lib
+
+    L = _lib.lib()
+    n = int(Fo.shape[0])
+    dev = Fo.device
+    stream = _lib.stream_handle(dev)
+    err = torch.empty((), dtype=torch.float64, device=dev)
+    if n <= L.asuka_scf_purify_max():
+        Fo = Fo.contiguous()
+        P = torch.empty((n, n), dtype=torch.float64, device=dev)
+        step = torch.empty((), dtype=torch.int32, device=dev)
+        _lib.check(L.asuka_scf_purify(_lib.ptr(Fo), n, int(nocc), int(iters), _PURIFY_TOL, _lib.ptr(P), _lib.ptr(err),
+                                      _lib.ptr(step), stream))
+        return P, err, lambda: int(step)
+    P = _purify_start(torch, Fo)
+    P2 = torch.empty_like(P)
+    work = torch.empty(256, dtype=torch.float64, device=dev)
+    done = torch.zeros(max(1, int(iters)), dtype=torch.int32, device=dev)
+    for it in range(int(iters)):
+        torch.matmul(P, P, out=P2)
+        _lib.check(L.asuka_scf_tc2_step(_lib.ptr(P), _lib.ptr(P2), n, int(nocc), _PURIFY_TOL, _lib.ptr(work),
+                                        _lib.ptr(done), it, _lib.ptr(err), stream))
+        if chunk and (it + 1) % chunk == 0 and int(done[it]):
+            break
+
+    def frozen_at():
+        k = np.nonzero(done.cpu().numpy())[0]
+        return int(k[0]) + 1 if k.size else 0
+
+    return _sym(P), err, frozen_at
+
+
 def _purify(torch, Fo, nocc: int, iters: int):
     """Projector onto the eigenvectors of the nocc lowest eigenvalues of the
     symmetric Fo, by trace-correcting purification (TC2; A. M. N. Niklasson,
@@ -361,42 +409,21 @@ def _purify(torch, Fo, nocc: int, iters: int):
     to 0 for a nonzero HOMO-LUMO gap. Each map repels one end of [0, 1] (P^2
     doubles the distance of eigenvalues below 1), so steps past convergence
     would undo it: once ||P^2 - P||_F falls below _PURIFY_TOL the projector is
-    frozen (a sticky device flag). Matrix products only, and the branch and the
-    freeze are device-side selects, so a fixed number of steps can be captured
-    in a HIP graph. Returns P and the idempotency error of the returned P."""
-    n = int(Fo.shape[0])
-    d = torch.diagonal(Fo)
-    r = Fo.abs().sum(dim=1) - d.abs()
-    e0 = (d - r).min()
-    e1 = (d + r).max()
-    eye = torch.eye(n, dtype=Fo.dtype, device=Fo.device)
-    P = (e1 * eye - Fo) / (e1 - e0)
-    done = torch.zeros((), dtype=torch.bool, device=Fo.device)
-    err = None
-    for _ in range(int(iters)):
-        P2 = P @ P
-        err = torch.linalg.norm(P2 - P)
-        done = done | (err < _PURIFY_TOL)
-        step = torch.where(torch.trace(P) > float(nocc), P2, 2.0 * P - P2)
-        P = torch.where(done, P, step)
-    return _sym(P), err
+    frozen (on the device). No host decisions, so a fixed number of steps can
+    be captured in a HIP graph. Returns P and the idempotency error of the
+    returned P."""
+    P, err, _ = _purify_run(torch, Fo, nocc, iters)
+    return P, err
 
 
-def _purify_steps(torch, Fo, nocc: int, max_steps: int = 300) -> int:
-    """Steps _purify takes on Fo until ||P^2 - P||_F < _PURIFY_TOL (eager, the
-    host reads the error every step)."""
-    n = int(Fo.shape[0])
-    d = torch.diagonal(Fo)
-    r = Fo.abs().sum(dim=1) - d.abs()
-    e0 = (d - r).min()
-    e1 = (d + r).max()
-    P = (e1 * torch.eye(n, dtype=Fo.dtype, device=Fo.device) - Fo) / (e1 - e0)
-    for k in range(1, max_steps + 1):
-        P2 = P @ P
-        if float(torch.linalg.norm(P2 - P)) < _PURIFY_TOL:
-            return k
-        P = P2 if float(torch.trace(P)) > nocc else 2.0 * P - P2
-    raise RuntimeError("density purification did not converge (no HOMO-LUMO gap?)")
+def _purify_converged(torch, Fo, nocc: int, max_steps: int = 300):
+    """(P, steps): the purified projector and the steps _purify takes on Fo until
+    ||P^2 - P||_F < _PURIFY_TOL (eager, the host reads the step count)."""
+    P, _, step = _purify_run(torch, Fo, nocc, max_steps, chunk=16)
+    k = step()
+    if k <= 0:
+        raise RuntimeError("density purification did not converge (no HOMO-LUMO gap?)")
+    return P, k
 
 
 def _rhf_graph_iterations(torch, S, h, X, D0, jk_ctx, *, F_probe=None, nocc, occ, enuc, max_cycle, conv_tol,
@@ -430,7 +457,7 @@ def _rhf_graph_iterations(torch, S, h, X, D0, jk_ctx, *, F_probe=None, nocc, occ
     # purification steps: measured on the last Fock matrix built before the
     # cycles (the predictor's; else one build of D0), with a margin
     F0 = F_probe if F_probe is not None else direct_fock_rhf(jk_ctx, D0, h, mixed_precision=mixed_precision)
-    npur = int(1.25 * _purify_steps(torch, _sym(X.T @ F0 @ X), nocc)) + 6
+    npur = int(1.25 * _purify_converged(torch, _sym(X.T @ F0 @ X), nocc)[1]) + 6
     nbuild = 1 if F_probe is None else 0  # Fock builds outside the cycles made here
 
     st = {

@@ -286,6 +286,26 @@ int asuka_int1e_grad(asuka_jk_ctx* ctx, const double* Dh, const double* Ws, doub
 int asuka_scf_diis_solve(const double* G, const int64_t* count, int nslot, double* coeff, int32_t* status,
                          void* stream);
 
+/* Density purification in place of eigh and aufbau (no counterpart in the
+ * reference, asuka/hf/df_scf.py:424-446): P (n x n, device) = the projector
+ * onto the eigenvectors of the nocc lowest eigenvalues of the symmetric F (n x
+ * n, device), by trace-correcting steps on the Gershgorin-scaled matrix, at
+ * most iters of them, stopped once ||P^2 - P||_F < tol. *err (device): that
+ * norm at the last step; *steps (device): the step it fell below tol, 0 if
+ * never. One kernel with the matrix in LDS: n <= asuka_scf_purify_max().
+ * Stream-ordered, graph-capturable. */
+int asuka_scf_purify_max(void);
+int asuka_scf_purify(const double* F, int n, int nocc, int iters, double tol, double* P, double* err, int32_t* steps,
+                     void* stream);
+
+/* One such step of a matrix of any size, with P2 = P P formed by the caller:
+ * P <- P2 if Tr P > nocc, else 2 P - P2, unless frozen: done[it] = (it > 0 and
+ * done[it - 1]) or ||P2 - P||_F < tol leaves P as it is. *err: that norm; work:
+ * 256 doubles of scratch; done: one int32 per step (all device memory).
+ * Stream-ordered, graph-capturable. */
+int asuka_scf_tc2_step(double* P, const double* P2, int n, int nocc, double tol, double* work, int32_t* done, int it,
+                       double* err, void* stream);
+
 /* ---- Density fitting: auxiliary metric and three-centre integrals ---- */
 typedef struct asuka_df_ctx asuka_df_ctx;
 
