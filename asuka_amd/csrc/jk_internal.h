@@ -56,8 +56,6 @@ enum EriMode : int {
   MODE_FOCK = 1,     // accumulate J - K/2 into F
   MODE_TILE = 2,     // write the tile
   MODE_SCHWARZ = 3,  // Q[P] = sqrt(max diag (P|P))
-  MODE_X3C = 4,      // three-centre (ab|P): X[P][a][b] (and [b][a]), ket pair = (aux shell, unit s)
-  MODE_V2C = 5,      // two-centre (P|Q): V[P][Q], bra and ket pairs = (aux shell, unit s)
 };
 
 // Device-side view of a context (passed by value to kernels).
@@ -176,10 +174,6 @@ struct ClassWork {
   const int* q_ab;
   const int* q_cd;
   const long long* q_out_off;
-  // product list (three- and two-centre integrals): work index k is the
-  // quartet (q_bra0 + k / q_nket, q_ket0 + k % q_nket) when q_nket > 0
-  long long q_nket;
-  int q_bra0, q_ket0;
   int cp_index;  // class-pair index (statistics counters)
   // mixed builds with routed units (the vote taken once per build before the
   // launches): the FP32 kernel's units and row tasks; units and tasks above
@@ -210,10 +204,6 @@ struct EriOut {
   const double* D2;
   double* J2;
   double* K2;
-  // MODE_X3C: X (x_naux, x_nao, x_nao); MODE_V2C: X (x_naux, x_naux); AO and
-  // auxiliary function indices are the shells' shell_ao
-  double* X;
-  long long x_nao, x_naux;
   // Ket-position buffers of the register kernels (null: J[c,d] by atomics on
   // J and D[c,d] read from D). Ket lists (col_pair) are laid out in blocks of
   // 64 positions of one ket class; block k holds component c (= ic * ND + id)
@@ -331,11 +321,6 @@ __device__ __forceinline__ double wave_total(double v) {
 // Decode work index k of a class pair into (bra pair, ket pair); false for
 // segment padding.
 __device__ inline bool decode_work(const ClassWork& w, long long k, int& P, int& Qp) {
-  if (w.q_nket > 0) {
-    P = w.q_bra0 + (int)(k / w.q_nket);
-    Qp = w.q_ket0 + (int)(k % w.q_nket);
-    return true;
-  }
   if (w.q_ab) {
     P = w.q_ab[k];
     Qp = w.q_cd[k];
