@@ -423,6 +423,57 @@ __global__ void k_route_tasks(const RowTask* __restrict__ tasks, long long ntask
   }
 }
 
+// Counters (EriOut::counters) of a class pair of the register kernels, one
+// wavefront per wave unit: what those kernels evaluate follows from the
+// screening alone, so they carry no counting code. f32: the units' precision
+// in mixed builds (null: all FP64).
+__global__ __launch_bounds__(256) void k_count_units(const DevBasis b, const WaveUnit* __restrict__ units,
+                                                     long long nunits, const int* __restrict__ f32,
+                                                     const int* __restrict__ col_pair, double eps_density,
+                                                     double eps_prim, unsigned long long* cnt) {
+  const int lane = threadIdx.x & 63;
+  for (long long k = blockIdx.x * 4LL + (threadIdx.x >> 6); k < nunits; k += gridDim.x * 4LL) {  // uniform per wave
+    const WaveUnit un = units[k];
+    const int P = un.P, pos = un.col + lane;
+    bool active = lane < (int)un.ncol;
+    if (active && eps_density > 0.0) active = (b.Q[P] * b.kq[pos]) * fmax(b.Dsp[P], b.kd[pos]) >= eps_density;
+    const int Qp = col_pair[active ? pos : un.col];
+    const UnitRange ur = unit_range(un, b.pp_count[P], false);
+    const bool first = active && ur.i0 == 0 && ur.j0 == 0;  // quartets are counted by their first slice
+    const int bin = ((b.sp_A[P] != b.sp_B[P]) << 2) | ((b.sp_A[Qp] != b.sp_B[Qp]) << 1) | (P != Qp);
+    for (int t = 0; t < 8; ++t) {
+      const unsigned long long m = __ballot(first && bin == t);
+      if (m && lane == 0) atomicAdd(cnt + t, (unsigned long long)__popcll(m));
+    }
+    const unsigned long long kq =
+        first ? (unsigned long long)b.pp_count0[P] * (unsigned long long)b.pp_count0[Qp] : 0ull;
+    const unsigned long long ksum = (unsigned long long)wave_total((double)kq);
+    const unsigned long long nact = (unsigned long long)__popcll(__ballot(first));
+    // primitive quartets the loops evaluate (after the primitive-quartet cut)
+    // and the lane slots the wave spends on them (64 x the longest lane)
+    long long nev = 0;
+    if (active && ur.ni > 0) {
+      const int cd0 = b.pp_start[Qp], ncd = min(b.pp_count[Qp], ur.j1);
+      const double kcut = eps_prim / b.ppf[b.pp_start[P] + ur.i0].q;
+      int j = ur.j0;
+      while (j < ncd && !(b.ppf[cd0 + j].q < kcut)) ++j;
+      nev = (long long)ur.ni * max(0, j - ur.j0);
+    }
+    const double nevs = wave_total((double)nev);
+    double nmax = (double)nev;
+    for (int off = 32; off > 0; off >>= 1) nmax = fmax(nmax, __shfl_xor(nmax, off));
+    if (lane == 0) {
+      atomicAdd(cnt + 8, ksum);
+      atomicAdd(cnt + 11, (unsigned long long)nevs);
+      atomicAdd(cnt + 12, 64ull * (unsigned long long)nmax);
+      if (f32 && f32[k]) {
+        atomicAdd(cnt + 9, nact);
+        atomicAdd(cnt + 10, ksum);
+      }
+    }
+  }
+}
+
 __global__ void k_rys_points(int n, long long npts, const double* T, double* x, double* w) {
   const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
   if (i >= npts) return;
@@ -648,10 +699,9 @@ static int pos_layout(asuka_jk_ctx* ctx, const std::vector<int>& col) {
       }
       kpoff[(size_t)k + 1] = kpoff[(size_t)k] + kmax;
     }
-    const long long nslot = std::max<long long>(1, kpoff.back() * 64);
-    if (nslot >= (1LL << 31)) return fail(ASUKA_E_INVALID, "ket primitive-pair table exceeds 2^31 slots");
-    std::vector<double> k64((size_t)(11 * nslot), 0.0), k32d((size_t)(3 * nslot), 0.0);
-    std::vector<float> k32f((size_t)(7 * nslot), 0.0f);
+    const size_t nrow = (size_t)std::max<long long>(1, kpoff.back());
+    std::vector<double> k64(nrow * 64 * kKet64, 0.0), k32d(nrow * 64 * kKet32d, 0.0);
+    std::vector<float> k32f(nrow * 64 * kKet32f, 0.0f);
     for (long long k = 0; k < nb; ++k)
       for (int t = 0; t < 64; ++t) {
         const int sp = col[(size_t)(k * 64 + t)];
@@ -659,16 +709,15 @@ static int pos_layout(asuka_jk_ctx* ctx, const std::vector<int>& col) {
         for (int j = 0; j < ctx->pp_count[sp]; ++j) {
           const PrimPairF& f = ctx->ppf[(size_t)ctx->pp_start[sp] + j];
           const double a_exp = ctx->pp[(size_t)ctx->pp_start[sp] + j].a_exp;
-          const size_t slot = (size_t)((kpoff[(size_t)k] + j) * 64 + t), n = (size_t)nslot;
-          const double v64[11] = {f.eta, f.inv_eta, f.ck, f.Px, f.Py, f.Pz, f.PAx, f.PAy, f.PAz, f.q, a_exp};
-          for (int x = 0; x < 11; ++x) k64[x * n + slot] = v64[x];
-          k32d[0 * n + slot] = f.Px;
-          k32d[1 * n + slot] = f.Py;
-          k32d[2 * n + slot] = f.Pz;
+          const size_t row = (size_t)(kpoff[(size_t)k] + j);
+          const double v64[kKet64] = {f.eta, f.inv_eta, f.ck, f.Px, f.Py, f.Pz, f.PAx, f.PAy, f.PAz, f.q, a_exp};
+          for (int x = 0; x < kKet64; ++x) k64[(row * kKet64 + x) * 64 + t] = v64[x];
+          const double v32d[kKet32d] = {f.Px, f.Py, f.Pz};
+          for (int x = 0; x < kKet32d; ++x) k32d[(row * kKet32d + x) * 64 + t] = v32d[x];
           // the same roundings as the FP32 pair table (q clamped to the float range)
-          const float v32[7] = {(float)f.eta, (float)f.inv_eta, (float)f.ck, (float)f.PAx, (float)f.PAy, (float)f.PAz,
-                                (float)std::min(f.q, 3e38)};
-          for (int x = 0; x < 7; ++x) k32f[x * n + slot] = v32[x];
+          const float v32[kKet32f] = {(float)f.eta, (float)f.inv_eta, (float)f.ck, (float)f.PAx, (float)f.PAy,
+                                      (float)f.PAz, (float)std::min(f.q, 3e38)};
+          for (int x = 0; x < kKet32f; ++x) k32f[(row * kKet32f + x) * 64 + t] = v32[x];
         }
       }
     long long* d_kpoff;
@@ -682,8 +731,8 @@ static int pos_layout(asuka_jk_ctx* ctx, const std::vector<int>& col) {
     ctx->dev.kp64 = d_k64;
     ctx->dev.kp32d = d_k32d;
     ctx->dev.kp32f = d_k32f;
-    ctx->dev.kslots = nslot;
   }
+  ctx->dev.pos_of_sp = ctx->d_pos_of_sp;
   ctx->dev.kq = ctx->d_qcol;
   ctx->dev.kd = ctx->d_kd;
   ctx->dev.kpp = d_kpp;
@@ -1690,6 +1739,12 @@ static int run_classes(asuka_jk_ctx* ctx, const EriOut& o, hipStream_t s, bool t
       if (bytes > ctx->lds_per_group - root_table_lds((w.la + w.lb + w.lc + w.ld) / 2 + 1) - 1024)
         w.acc_colsC = w.acc_colsD = 0;
     }
+    if (o.counters && cph.nunits > 0 && eri_fast_has_plan(w.la, w.lb, w.lc, w.ld)) {
+      hipLaunchKernelGGL(k_count_units, dim3(grid_for(cph.nunits, 4)), dim3(256), 0, ls, *dev,
+                         ctx->d_units + cph.unit_start, cph.nunits, routed ? ctx->d_rf32 + cph.unit_start : nullptr,
+                         ctx->d_col_pair, o.eps_density, o.eps_prim, o.counters + (size_t)kCountStride * i);
+      HIP_CHECK(hipGetLastError());
+    }
     bool handled = false;
     HIP_CHECK(launch_eri_fast(*dev, w, oo, ls, &handled));
     if (!handled) HIP_CHECK(launch_eri_coop(*dev, w, o, ls, &handled));
@@ -2019,6 +2074,15 @@ int asuka_jk_autotune(asuka_jk_ctx* ctx, const double* D, int flags, int reps, v
   o.eps_prim = ctx->eps_schwarz > 0.0 ? ctx->eps_prim : 0.0;
   o.mixed = (flags & ASUKA_JK_MIXED) ? 1 : 0;
   o.tau_mixed = ctx->tau_mixed;
+  if (ctx->nblk > 0) {  // the ket-position and flush buffers, as in a build (their contents are discarded)
+    o.jblk = ctx->d_jblk;
+    o.Jpos = ctx->d_jpos;
+    o.Dpos = ctx->d_dpos;
+    o.Kc = ctx->d_kc;
+    hipLaunchKernelGGL(k_pos_gather, dim3((unsigned)ctx->nblk), dim3(64), 0, s, ctx->dev, ctx->d_col_pair, ctx->d_jblk,
+                       D, nullptr, ctx->d_dpos, ctx->d_jpos, ctx->pos_len);
+    HIP_CHECK(hipGetLastError());
+  }
   // median of reps timed launches (after one untimed) of class pair i as it is now set up
   auto time_class = [&](int i, double* ms) -> int {
     std::vector<float> t;

@@ -187,47 +187,119 @@ __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlan
 __device__ __forceinline__ double wave_sum(double v) { return wave_total(v); }
 
 
-// The ket primitive pair in slot t of the transposed tables (DevBasis::kpoff):
-// the field bases are wave-uniform and the slot a 32-bit per-lane offset, so
-// each field is one load with a scalar base and a vector offset.
-template <typename PPT>
-__device__ __forceinline__ PPT load_ket(const DevBasis& b, int t);
-template <>
-__device__ __forceinline__ PrimPairF load_ket<PrimPairF>(const DevBasis& b, int t) {
-  const double* k = b.kp64;
-  const long long n = b.kslots;
-  PrimPairF y;
-  y.eta = k[t];
-  y.inv_eta = (k + n)[t];
-  y.ck = (k + 2 * n)[t];
-  y.Px = (k + 3 * n)[t];
-  y.Py = (k + 4 * n)[t];
-  y.Pz = (k + 5 * n)[t];
-  y.PAx = (k + 6 * n)[t];
-  y.PAy = (k + 7 * n)[t];
-  y.PAz = (k + 8 * n)[t];
-  y.q = (k + 9 * n)[t];
-  return y;
+// Everything the kernels below read is passed in one struct by value and
+// fetched from the kernel-argument segment where it is used (ArgP), not held
+// in scalar registers: with three argument structs and their pointers live
+// across the item loop the compiler spilled about 160 scalar registers to
+// lanes of vector registers and moved them back all over an item ((10|10)
+// FP64: 164 spills, 3504 instructions, 137 VGPRs; now 24, 1838 and 109).
+// refetch() hides the pointer's origin so that loads through it are not
+// hoisted over it. Measured, with the bra's rows as uniform bases, the next bra
+// primitive pair in flight and the counting code in a kernel of its own:
+// (H2O)27 cc-pVDZ FP64 Fock build 62.9 -> 55.5 ms, (H2O)64 mixed 331 -> 299 ms,
+// batch of 14 clusters 30.4 -> 25.4 ms, (H2O)8 cc-pVTZ mixed 56.7 -> 52.8 ms.
+// One density of a build: where it is read and what it is digested into
+// (null: not wanted). D, J and K of MODE_FOCK builds: J = K = F.
+struct FastDen {
+  const double* D;
+  double* J;
+  double* K;
+  const double* Dpos;  // EriOut::jblk
+  double* Jpos;
+  double* Kc;
+};
+struct FastArgs {
+  const WaveUnit* units;
+  const RowTask* tasks;
+  unsigned int* queue;
+  const void* pp;       // bra primitive pairs: PrimPairF, or PrimPairF32 for the FP32 kernels
+  const double* kpd;    // ket primitive pairs (DevBasis::kpoff) of this precision
+  const float* kpf;
+  const long long* kpoff;
+  const int *sp_A, *sp_B, *pp_start, *pp_count, *shell_ao, *shell_mol, *mol_n, *mol_lao, *lao_ao, *pos_of_sp;
+  const long long *mol_shift, *jblk;
+  const double *shell_xyz, *Q, *Dsp, *kq, *kd, *kcd;
+  const int2 *kpp, *kao, *klao;
+  FastDen den[2];
+  double eps_density, eps_prim, tau_mixed;
+  double ks;  // factor of the K sums: 1, or -1/2 for MODE_FOCK
+  int nden, ntasks, wpg, vote;  // vote: each kernel takes the units of its precision (mixed builds without routed lists)
+  int acc_colsC, acc_colsD, lao_offC, lao_offD;
+};
+#define ASUKA_CONST __attribute__((address_space(4)))
+#define ASUKA_GLOB __attribute__((address_space(1)))
+using ArgP = const ASUKA_CONST FastArgs*;
+__device__ __forceinline__ ArgP refetch(ArgP p) {
+  asm volatile("" : "+s"(p));
+  return p;
 }
-template <>
-__device__ __forceinline__ PrimPairF32 load_ket<PrimPairF32>(const DevBasis& b, int t) {
-  const double* d = b.kp32d;
-  const float* f = b.kp32f;
-  const long long n = b.kslots;
-  PrimPairF32 y;
-  y.Px = d[t];
-  y.Py = (d + n)[t];
-  y.Pz = (d + 2 * n)[t];
-  y.eta = f[t];
-  y.inv_eta = (f + n)[t];
-  y.ck = (f + 2 * n)[t];
-  y.PAx = (f + 3 * n)[t];
-  y.PAy = (f + 4 * n)[t];
-  y.PAz = (f + 5 * n)[t];
-  y.q = (f + 6 * n)[t];
-  y.pad = 0.0f;
-  return y;
+// Read-only tables at wave-uniform indices: scalar loads.
+template <typename T>
+__device__ __forceinline__ T cl(const T* p, long long i) {
+  return ((const ASUKA_CONST T*)p)[i];
 }
+// A wave-uniform base and a 32-bit byte offset per lane.
+template <typename T>
+__device__ __forceinline__ T gl(const void* base, unsigned off) {
+  return *(const ASUKA_GLOB T*)((const ASUKA_GLOB char*)base + off);
+}
+typedef int i32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+// A primitive pair in the arithmetic CT of the recursion; P stays FP64 so that
+// P - Q is formed in FP64.
+template <typename CT>
+struct Prim {
+  double Px, Py, Pz;
+  CT eta, ieta, ck, ax, ay, az, q;
+};
+template <typename CT>
+__device__ __forceinline__ Prim<CT> load_bra(const void* pp, int i) {  // i uniform
+  Prim<CT> r;
+  if constexpr (sizeof(CT) == 8) {
+    const ASUKA_CONST double* d = (const ASUKA_CONST double*)pp + (sizeof(PrimPairF) / 8) * (long long)i;
+    r.eta = d[0], r.ieta = d[1], r.ck = d[2], r.Px = d[3], r.Py = d[4], r.Pz = d[5];
+    r.ax = d[6], r.ay = d[7], r.az = d[8];
+  } else {
+    const ASUKA_CONST double* d = (const ASUKA_CONST double*)pp + (sizeof(PrimPairF32) / 8) * (long long)i;
+    const ASUKA_CONST float* f = (const ASUKA_CONST float*)(d + 3);
+    r.Px = d[0], r.Py = d[1], r.Pz = d[2];
+    r.eta = f[0], r.ieta = f[1], r.ck = f[2], r.ax = f[3], r.ay = f[4], r.az = f[5];
+  }
+  r.q = CT(0);
+  return r;
+}
+// The lane's primitive pair of slot row s of the ket tables (DevBasis::kpoff):
+// one scalar base, the fields at immediate offsets.
+template <typename CT>
+__device__ __forceinline__ Prim<CT> load_ket(const double* kpd, const float* kpf, long long s, unsigned lane) {
+  Prim<CT> r;
+  if constexpr (sizeof(CT) == 8) {
+    const double* k = kpd + s * (64 * kKet64);
+    r.eta = gl<double>(k, 8 * lane), r.ieta = gl<double>(k, 8 * lane + 512), r.ck = gl<double>(k, 8 * lane + 1024);
+    r.Px = gl<double>(k, 8 * lane + 1536), r.Py = gl<double>(k, 8 * lane + 2048), r.Pz = gl<double>(k, 8 * lane + 2560);
+    r.ax = gl<double>(k, 8 * lane + 3072), r.ay = gl<double>(k, 8 * lane + 3584);
+    r.az = gl<double>(k + 512, 8 * lane), r.q = gl<double>(k + 512, 8 * lane + 512);
+  } else {
+    const double* k = kpd + s * (64 * kKet32d);
+    const float* f = kpf + s * (64 * kKet32f);
+    r.Px = gl<double>(k, 8 * lane), r.Py = gl<double>(k, 8 * lane + 512), r.Pz = gl<double>(k, 8 * lane + 1024);
+    r.eta = gl<float>(f, 4 * lane), r.ieta = gl<float>(f, 4 * lane + 256), r.ck = gl<float>(f, 4 * lane + 512);
+    r.ax = gl<float>(f, 4 * lane + 768), r.ay = gl<float>(f, 4 * lane + 1024), r.az = gl<float>(f, 4 * lane + 1280);
+    r.q = gl<float>(f, 4 * lane + 1536);
+  }
+  return r;
+}
+
+// The bra pair of a row task (uniform).
+struct Bra {
+  int P, ab0;      // shell pair, its first primitive pair
+  int A, B;        // shells
+  int aoA, aoB;    // first AOs
+  int posP;        // the pair's own ket position, -1 if it has none
+  int N;           // row stride of the molecule's D/J/K block
+  long long msh;   // element offset of that block (mol_layout)
+};
 
 // Arithmetic helpers for the compute type CT of the recursion (double, or
 // float on the FP32 path).
@@ -258,24 +330,21 @@ struct RowAcc {
   int stride;  // offset of the second density's accumulators (two-density builds)
 };
 
-// One chunk of one shell quartet per lane; the bra pair P is the same on every
+// One chunk of one shell quartet per lane; the bra pair is the same on every
 // lane of the wave (bra-uniform wave units), so the bra primitive pairs are
 // read with scalar loads in the inner loop while each lane streams its own
 // ket primitive pairs in the outer loop. CT is the type of the primitive
 // setup, roots, VRR, contracted intermediates and HRR; the digestion always
 // accumulates in FP64. Geometric differences are formed in FP64 and rounded.
 // `tab` is the NR-root block of the root table in CT (LDS or global).
+// col: the unit's first ket position (uniform; a 64-position block boundary).
 // jcd: with the plan split over A components, the J[c,d] partial sums of the
 // first density over this chunk's A components are added into jcd (the
 // lane's registers, NCL*ND values) and the caller issues one atomic per
 // element after the last A chunk; nullptr: atomics here.
-// jb: the unit's block in the ket-position buffers (EriOut::jblk; uniform),
-// or -1 for D[c,d] from D and J[c,d] atomics on J.
-
 template <class PL, int CH, typename CT, bool FX>
-__device__ __forceinline__ void run_chunk(const DevBasis& b, const EriOut& o, int P, int Qp, int pos,
-                                          const UnitRange& ur, bool active, const CT* __restrict__ tab, const RowAcc& acc, double* jcd,
-                                          long long jb) {
+__device__ __forceinline__ void run_chunk(ArgP ap, const Bra& br, int col, const UnitRange& ur, bool active,
+                                          const CT* __restrict__ tab, const RowAcc& acc, double* jcd) {
   using CK = Chunk<PL, CH>;
   constexpr int NEL = CK::NEL, NFL = CK::NFL, NR = PL::NR;
   constexpr int NMAX = PL::NMAX, MMAX = PL::MMAX;
@@ -288,23 +357,11 @@ __device__ __forceinline__ void run_chunk(const DevBasis& b, const EriOut& o, in
   constexpr auto tf = PL::RF::tab();
   constexpr auto L = CK::L;
   const CT one = CT(1), half = CT(0.5);
+  const unsigned lane = threadIdx.x & 63;
 
-  // bra-side indices are wave-uniform; readfirstlane states it so that the
-  // loads addressed by them are scalar
-  // the ket pair's data by its position (pos: contiguous across the lanes)
-  const int A = uni(b.sp_A[P]), B = uni(b.sp_B[P]);
-  const double Ax = b.shell_xyz[3 * A], Ay = b.shell_xyz[3 * A + 1], Az = b.shell_xyz[3 * A + 2];
-  const int ab0 = uni(b.pp_start[P]) + ur.i0, nab = ur.ni;  // the unit's bra primitive pairs
-  const int2 kpp = b.kpp[pos];
-  const int ncd = active ? min(kpp.y, ur.j1) : 0;  // (kpp.x, the first pair in the pair table, is for host-side use)
-  // the primitive pairs in the precision of CT (the FP32 path reads the float
-  // copy: no conversions in the primitive loop but P - Q, formed in FP64)
-  using PPT = typename std::conditional<sizeof(CT) == 4, PrimPairF32, PrimPairF>::type;
-  const PPT* __restrict__ ppf;
-  if constexpr (sizeof(CT) == 4)
-    ppf = b.ppf32;
-  else
-    ppf = b.ppf;
+  ap = refetch(ap);
+  const int ab0 = br.ab0 + ur.i0, nab = ur.ni;  // the unit's bra primitive pairs
+  const int ncd = active ? min(gl<int>(ap->kpp + col, 8 * lane + 4), ur.j1) : 0;
 
   CT ef[NEL * NFL];
 #pragma unroll
@@ -316,28 +373,37 @@ __device__ __forceinline__ void run_chunk(const DevBasis& b, const EriOut& o, in
   // ket-pair bound of the unit is below eps_prim; a lane leaves its ket loop
   // at the first ket pair whose q times the largest bra bound is below it.
   // Every skipped primitive quartet adds less than eps_prim to each integral.
-  const CT kcut = (nab > 0 && o.eps_prim > 0.0) ? CT(o.eps_prim / (double)ppf[ab0].q) : CT(0);
-  // the lane's ket primitive pairs, transposed by position (the lanes' j-th
-  // pairs are contiguous): slots ks0 + 64 j
-  const int ks0 = (int)b.kpoff[uni(pos >> 6)] * 64 + (pos & 63);
-  PPT Yn;
-  if (ur.j0 < ncd) Yn = load_ket<PPT>(b, ks0 + 64 * ur.j0);
-  for (int j = ur.j0; j < ncd; ++j) {
-    const PPT Y = Yn;
-    if (Y.q < kcut) break;  // per lane: the rest of its ket pairs are smaller
-    if (j + 1 < ncd) Yn = load_ket<PPT>(b, ks0 + 64 * (j + 1));  // next ket pair, in flight during this one
-    const CT q = CT(Y.eta), iq = CT(Y.inv_eta), ckq = CT(Y.ck);
-    const CT QCx = CT(Y.PAx), QCy = CT(Y.PAy), QCz = CT(Y.PAz);
-    for (int i = 0; i < nab; ++i) {
-      const PPT X = ppf[ab0 + i];  // wave-uniform
-      const CT p = CT(X.eta), ip = CT(X.inv_eta);
-      const CT PAx = CT(X.PAx), PAy = CT(X.PAy), PAz = CT(X.PAz);
+  if (nab > 0) {
+    const void* pp = ap->pp;
+    const double* kpd = ap->kpd;
+    const float* kpf = ap->kpf;
+    CT kcut;
+    if constexpr (sizeof(CT) == 8)
+      kcut = ap->eps_prim * rcp_nr(((const ASUKA_CONST PrimPairF*)pp)[ab0].q);
+    else
+      kcut = CT(ap->eps_prim * rcp_nr((double)((const ASUKA_CONST PrimPairF32*)pp)[ab0].q));
+    // slot rows of the unit's block: the lanes' j-th primitive pairs
+    const long long ks0 = cl(ap->kpoff, col >> 6);
+    Prim<CT> Yn;
+    if (ur.j0 < ncd) Yn = load_ket<CT>(kpd, kpf, ks0 + ur.j0, lane);
+    Prim<CT> X = load_bra<CT>(pp, ab0);
+    for (int j = ur.j0; j < ncd; ++j) {
+      const Prim<CT> Y = Yn;
+      if (Y.q < kcut) break;  // per lane: the rest of its ket pairs are smaller
+      if (j + 1 < ncd) Yn = load_ket<CT>(kpd, kpf, ks0 + uni(j + 1), lane);  // next ket pair, in flight during this one
+      const CT q = Y.eta, iq = Y.ieta, ckq = Y.ck;
+      const CT QCx = Y.ax, QCy = Y.ay, QCz = Y.az;
+      for (int i = 0; i < nab; ++i) {
+        // the next bra pair (wave-uniform; the first again for the next ket pair) is in flight during this one
+        const Prim<CT> Xn = load_bra<CT>(pp, ab0 + (i + 1 < nab ? i + 1 : 0));
+      const CT p = X.eta, ip = X.ieta;
+      const CT PAx = X.ax, PAy = X.ay, PAz = X.az;
       const CT spq = p + q;
       const CT inv_pq = rcp_nr(spq);
       const CT dx = CT(X.Px - Y.Px), dy = CT(X.Py - Y.Py), dz = CT(X.Pz - Y.Pz);
       const CT T = p * q * inv_pq * (dx * dx + dy * dy + dz * dz);
       // 2 pi^(5/2) cK_ab cK_cd / (p q sqrt(p+q))
-      const CT base = CT(X.ck) * ckq * rsq_nr(spq);
+      const CT base = X.ck * ckq * rsq_nr(spq);
       CT rx[NR], rw[NR];
       rys_roots_blk<NR, CT, (NR <= kLdsRootsMax ? rys_c::lds_stride_of<CT>(NR) : rys_c::interval_size_of<CT>(NR))>(
           T, tab, rx, rw);
@@ -381,15 +447,21 @@ __device__ __forceinline__ void run_chunk(const DevBasis& b, const EriOut& o, in
           }
         }
       }
+        X = Xn;
+      }
     }
   }
 
   // ---- horizontal transfer: ket (C-components of the chunk) then bra ----
-  const double Bx = b.shell_xyz[3 * B], By = b.shell_xyz[3 * B + 1], Bz = b.shell_xyz[3 * B + 2];
+  ap = refetch(ap);
   CT pab[3][LB + 1], pcd[3][LD + 1];
   {
-    const CT ab[3] = {CT(Ax - Bx), CT(Ay - By), CT(Az - Bz)};
-    const CT cd[3] = {CT(b.kcd[3 * pos]), CT(b.kcd[3 * pos + 1]), CT(b.kcd[3 * pos + 2])};
+    CT ab[3], cd[3];
+#pragma unroll
+    for (int ax = 0; ax < 3; ++ax) {
+      ab[ax] = LB > 0 ? CT(cl(ap->shell_xyz, 3 * br.A + ax) - cl(ap->shell_xyz, 3 * br.B + ax)) : CT(0);
+      cd[ax] = LD > 0 ? CT(gl<double>(ap->kcd + 3 * (long long)col, 24 * lane + 8 * ax)) : CT(0);
+    }
 #pragma unroll
     for (int ax = 0; ax < 3; ++ax) {
       pab[ax][0] = one;
@@ -452,52 +524,46 @@ __device__ __forceinline__ void run_chunk(const DevBasis& b, const EriOut& o, in
   // workgroup's LDS accumulators when present (flushed once per row task),
   // J[c,d] (distinct per lane) to global atomics. With a second density
   // (two-density builds) the same tile is digested again into (J2, K2).
-  long long N, msh;  // the molecule's D/J/K block (uniform: the bra pair is)
-  mol_layout(b, A, N, msh);
-  const int2 kao = b.kao[pos];
-  const int aoA = b.shell_ao[A] + a0, aoB = b.shell_ao[B], aoC = kao.x + c0, aoD = kao.y;
-  const bool ab_neq = A != B, cd_neq = kao.x != kao.y, bk = P != Qp;
+  const int N = br.N;
+  const i32x2 kao = gl<i32x2>(ap->kao + col, 8 * lane);
+  const unsigned oC = 8u * (unsigned)(kao.x + c0), oD = 8u * (unsigned)kao.y;  // byte offsets of the lane's columns
+  const bool ab_neq = br.A != br.B, cd_neq = kao.x != kao.y, bk = br.posP != col + (int)lane;
   const double fj = (ab_neq ? 2.0 : 1.0) * (cd_neq ? 2.0 : 1.0);
-  const double fk = bk ? 2.0 : 1.0;
-  const double ks = (o.mode == MODE_FOCK) ? -0.5 * fk : fk;
+  const double ks = bk ? 2.0 * ap->ks : ap->ks;
   const bool lds = acc.on;  // uniform
   // compact columns of the lane's C (first component of the chunk) and D shells
-  const int2 klao = b.klao[pos];
-  const int colC = lds ? klao.x + c0 : 0, colD = lds ? klao.y : 0;
-  const int nden = o.D2 ? 2 : 1;  // uniform
+  const i32x2 klao = gl<i32x2>(ap->klao + col, 8 * lane);
+  const int colC = klao.x + c0, colD = klao.y;
+  const int nden = ap->nden;  // uniform
   for (int di = 0; di < nden; ++di) {
-    const double* Dm = (di ? o.D2 : o.D) + msh;
-    double* Jo = shifted(di ? o.J2 : ((o.mode == MODE_FOCK) ? o.F : o.J), msh);
-    double* Ko = shifted(di ? o.K2 : ((o.mode == MODE_FOCK) ? o.F : o.K), msh);
+    const ASUKA_CONST FastDen* dn = &ap->den[di];
+    const double* Dm = dn->D + br.msh;
+    double* Jo = dn->J;
     const int so = di * acc.stride;  // this density's accumulators in s_acc
+    // rows of the bra's AOs (uniform bases)
+    auto rowA = [&](int ia) { return Dm + (long long)(br.aoA + a0 + ia) * N; };
+    auto rowB = [&](int ib) { return Dm + (long long)(br.aoB + ib) * N; };
     if (Jo) {
-      const int lane = threadIdx.x & 63;
-      double dcd[NCDL];
-      if (jb >= 0) {  // the chunk's components c0 * ND.. of the lane's ket position
-        const double* Dp = (di ? o.Dpos2 : o.Dpos) + jb + 64LL * (c0 * ND) + lane;
+      const long long jb = cl(ap->jblk, col >> 6) + 64LL * (c0 * ND);  // the chunk's components of the unit's block
+      {
+        double dcd[NCDL];
+        const double* Dp = dn->Dpos + jb;
 #pragma unroll
-        for (int c = 0; c < NCDL; ++c) dcd[c] = Dp[64 * c];
-      } else {
+        for (int c = 0; c < NCDL; ++c) dcd[c] = gl<double>(Dp, 8 * lane + 512 * c);
+        // The bra pair, hence the J[a,b] addresses, is the same on every lane:
+        // reduce across the wave, one update per element.
 #pragma unroll
-        for (int ic = 0; ic < NCL; ++ic)
+        for (int r = 0; r < NAL * NB; ++r) {
+          double s = 0.0;
 #pragma unroll
-          for (int id = 0; id < ND; ++id) dcd[ic * ND + id] = Dm[(aoC + ic) * N + aoD + id];
-      }
-      // The bra pair, hence the J[a,b] addresses, is the same on every lane:
-      // reduce across the wave, one update per element.
-      const unsigned long long amask = __ballot(active);
-      const int first = amask ? (__ffsll((unsigned long long)amask) - 1) : 0;
-#pragma unroll
-      for (int r = 0; r < NAL * NB; ++r) {
-        double s = 0.0;
-#pragma unroll
-        for (int c = 0; c < NCDL; ++c) s = fma((double)tile[r * NCDL + c], dcd[c], s);
-        s = wave_sum(active ? fj * s : 0.0);
-        if (lane == first && active) {
-          if (lds)
-            acc_add(&s_acc[so + acc.jab + (a0 + r / NB) * NB + r % NB], s, FX);
-          else
-            acc_add(&Jo[(aoA + r / NB) * N + aoB + r % NB], s, FX);
+          for (int c = 0; c < NCDL; ++c) s = fma((double)tile[r * NCDL + c], dcd[c], s);
+          s = wave_sum(active ? fj * s : 0.0);
+          if (lane == 0) {
+            if (lds)
+              acc_add(&s_acc[so + acc.jab + (a0 + r / NB) * NB + r % NB], s, FX);
+            else
+              acc_add(Jo + br.msh + (long long)(br.aoA + a0 + r / NB) * N + br.aoB + r % NB, s, FX);
+          }
         }
       }
       if (bk && active) {
@@ -505,7 +571,8 @@ __device__ __forceinline__ void run_chunk(const DevBasis& b, const EriOut& o, in
 #pragma unroll
         for (int ia = 0; ia < NAL; ++ia)
 #pragma unroll
-          for (int ib = 0; ib < NB; ++ib) dab[ia * NB + ib] = Dm[(aoA + ia) * N + aoB + ib];
+          for (int ib = 0; ib < NB; ++ib) dab[ia * NB + ib] = cl(rowA(ia), br.aoB + ib);
+        double* Jp = dn->Jpos + jb;
 #pragma unroll
         for (int c = 0; c < NCDL; ++c) {
           double s = 0.0;
@@ -513,20 +580,25 @@ __device__ __forceinline__ void run_chunk(const DevBasis& b, const EriOut& o, in
           for (int r = 0; r < NAL * NB; ++r) s = fma((double)tile[r * NCDL + c], dab[r], s);
           if (jcd && di == 0)
             jcd[c] = fma(fj, s, jcd[c]);
-          else if (jb >= 0)
-            acc_add((di ? o.Jpos2 : o.Jpos) + jb + 64LL * (c0 * ND + c) + lane, fj * s, FX);
           else
-            acc_add(&Jo[(aoC + c / ND) * N + aoD + c % ND], fj * s, FX);
+            acc_add((double*)((ASUKA_GLOB char*)Jp + (8 * lane + 512 * c)), fj * s, FX);
         }
       }
     }
+    double* Ko = dn->K;
     if (Ko && active) {
+      auto addK = [&](int off, int cols, int col0, long long row, unsigned o, double v) {
+        if (lds)
+          acc_add(&s_acc[so + off + cols + col0], v, FX);
+        else
+          acc_add((double*)((ASUKA_GLOB char*)(Ko + br.msh + row * N) + o), v, FX);
+      };
       {  // K[a,c] += sum_{b,d} v D[b,d]
         double dbd[NB * ND];
 #pragma unroll
         for (int ib = 0; ib < NB; ++ib)
 #pragma unroll
-          for (int id = 0; id < ND; ++id) dbd[ib * ND + id] = Dm[(aoB + ib) * N + aoD + id];
+          for (int id = 0; id < ND; ++id) dbd[ib * ND + id] = gl<double>(rowB(ib), oD + 8 * id);
 #pragma unroll
         for (int ia = 0; ia < NAL; ++ia)
 #pragma unroll
@@ -536,10 +608,7 @@ __device__ __forceinline__ void run_chunk(const DevBasis& b, const EriOut& o, in
             for (int ib = 0; ib < NB; ++ib)
 #pragma unroll
               for (int id = 0; id < ND; ++id) s = fma((double)tile[(ia * NB + ib) * NCDL + ic * ND + id], dbd[ib * ND + id], s);
-            if (lds)
-              acc_add(&s_acc[so + acc.kac + (a0 + ia) * acc.colsC + colC + ic], ks * s, FX);
-            else
-              acc_add(&Ko[(aoA + ia) * N + aoC + ic], ks * s, FX);
+            addK(acc.kac, (a0 + ia) * acc.colsC, colC + ic, br.aoA + a0 + ia, oC + 8 * ic, ks * s);
           }
       }
       if (cd_neq) {  // K[a,d] += sum_{b,c} v D[b,c]
@@ -547,7 +616,7 @@ __device__ __forceinline__ void run_chunk(const DevBasis& b, const EriOut& o, in
 #pragma unroll
         for (int ib = 0; ib < NB; ++ib)
 #pragma unroll
-          for (int ic = 0; ic < NCL; ++ic) dbc[ib * NCL + ic] = Dm[(aoB + ib) * N + aoC + ic];
+          for (int ic = 0; ic < NCL; ++ic) dbc[ib * NCL + ic] = gl<double>(rowB(ib), oC + 8 * ic);
 #pragma unroll
         for (int ia = 0; ia < NAL; ++ia)
 #pragma unroll
@@ -557,10 +626,7 @@ __device__ __forceinline__ void run_chunk(const DevBasis& b, const EriOut& o, in
             for (int ib = 0; ib < NB; ++ib)
 #pragma unroll
               for (int ic = 0; ic < NCL; ++ic) s = fma((double)tile[(ia * NB + ib) * NCDL + ic * ND + id], dbc[ib * NCL + ic], s);
-            if (lds)
-              acc_add(&s_acc[so + acc.kad + (a0 + ia) * acc.colsD + colD + id], ks * s, FX);
-            else
-              acc_add(&Ko[(aoA + ia) * N + aoD + id], ks * s, FX);
+            addK(acc.kad, (a0 + ia) * acc.colsD, colD + id, br.aoA + a0 + ia, oD + 8 * id, ks * s);
           }
       }
       if (ab_neq) {  // K[b,c] += sum_{a,d} v D[a,d]
@@ -568,7 +634,7 @@ __device__ __forceinline__ void run_chunk(const DevBasis& b, const EriOut& o, in
 #pragma unroll
         for (int ia = 0; ia < NAL; ++ia)
 #pragma unroll
-          for (int id = 0; id < ND; ++id) dad[ia * ND + id] = Dm[(aoA + ia) * N + aoD + id];
+          for (int id = 0; id < ND; ++id) dad[ia * ND + id] = gl<double>(rowA(ia), oD + 8 * id);
 #pragma unroll
         for (int ib = 0; ib < NB; ++ib)
 #pragma unroll
@@ -578,17 +644,14 @@ __device__ __forceinline__ void run_chunk(const DevBasis& b, const EriOut& o, in
             for (int ia = 0; ia < NAL; ++ia)
 #pragma unroll
               for (int id = 0; id < ND; ++id) s = fma((double)tile[(ia * NB + ib) * NCDL + ic * ND + id], dad[ia * ND + id], s);
-            if (lds)
-              acc_add(&s_acc[so + acc.kbc + ib * acc.colsC + colC + ic], ks * s, FX);
-            else
-              acc_add(&Ko[(aoB + ib) * N + aoC + ic], ks * s, FX);
+            addK(acc.kbc, ib * acc.colsC, colC + ic, br.aoB + ib, oC + 8 * ic, ks * s);
           }
         if (cd_neq) {  // K[b,d] += sum_{a,c} v D[a,c]
           double dac[NAL * NCL];
 #pragma unroll
           for (int ia = 0; ia < NAL; ++ia)
 #pragma unroll
-            for (int ic = 0; ic < NCL; ++ic) dac[ia * NCL + ic] = Dm[(aoA + ia) * N + aoC + ic];
+            for (int ic = 0; ic < NCL; ++ic) dac[ia * NCL + ic] = gl<double>(rowA(ia), oC + 8 * ic);
 #pragma unroll
           for (int ib = 0; ib < NB; ++ib)
 #pragma unroll
@@ -599,10 +662,7 @@ __device__ __forceinline__ void run_chunk(const DevBasis& b, const EriOut& o, in
 #pragma unroll
                 for (int ic = 0; ic < NCL; ++ic)
                   s = fma((double)tile[(ia * NB + ib) * NCDL + ic * ND + id], dac[ia * NCL + ic], s);
-              if (lds)
-                acc_add(&s_acc[so + acc.kbd + ib * acc.colsD + colD + id], ks * s, FX);
-              else
-                acc_add(&Ko[(aoB + ib) * N + aoD + id], ks * s, FX);
+              addK(acc.kbd, ib * acc.colsD, colD + id, br.aoB + ib, oD + 8 * id, ks * s);
             }
         }
       }
@@ -611,26 +671,24 @@ __device__ __forceinline__ void run_chunk(const DevBasis& b, const EriOut& o, in
 }
 
 template <class PL, int CH, typename CT, bool FX>
-__device__ __forceinline__ void dispatch_chunk(int chunk, const DevBasis& b, const EriOut& o, int P, int Qp, int pos,
-                                               const UnitRange& ur, bool active, const CT* __restrict__ tab, const RowAcc& acc,
-                                               long long jb) {
+__device__ __forceinline__ void dispatch_chunk(int chunk, ArgP ap, const Bra& br, int col, const UnitRange& ur,
+                                               bool active, const CT* __restrict__ tab, const RowAcc& acc) {
   if constexpr (CH < PL::NCH) {
     if (chunk == CH) {
-      run_chunk<PL, CH, CT, FX>(b, o, P, Qp, pos, ur, active, tab, acc, nullptr, jb);
+      run_chunk<PL, CH, CT, FX>(ap, br, col, ur, active, tab, acc, nullptr);
       return;
     }
-    dispatch_chunk<PL, CH + 1, CT, FX>(chunk, b, o, P, Qp, pos, ur, active, tab, acc, jb);
+    dispatch_chunk<PL, CH + 1, CT, FX>(chunk, ap, br, col, ur, active, tab, acc);
   }
 }
 
 // The A chunks CA.. of C chunk CC, in sequence, carrying J[c,d] in jcd.
 template <class PL, int CC, int CA, typename CT, bool FX>
-__device__ __forceinline__ void run_agroup(const DevBasis& b, const EriOut& o, int P, int Qp, int pos,
-                                           const UnitRange& ur, bool active, const CT* __restrict__ tab, const RowAcc& acc, double* jcd,
-                                           long long jb) {
+__device__ __forceinline__ void run_agroup(ArgP ap, const Bra& br, int col, const UnitRange& ur, bool active,
+                                           const CT* __restrict__ tab, const RowAcc& acc, double* jcd) {
   if constexpr (CA < PL::SPLIT_A) {
-    run_chunk<PL, CA * PL::SPLIT_C + CC, CT, FX>(b, o, P, Qp, pos, ur, active, tab, acc, jcd, jb);
-    run_agroup<PL, CC, CA + 1, CT, FX>(b, o, P, Qp, pos, ur, active, tab, acc, jcd, jb);
+    run_chunk<PL, CA * PL::SPLIT_C + CC, CT, FX>(ap, br, col, ur, active, tab, acc, jcd);
+    run_agroup<PL, CC, CA + 1, CT, FX>(ap, br, col, ur, active, tab, acc, jcd);
   }
 }
 
@@ -638,96 +696,59 @@ __device__ __forceinline__ void run_agroup(const DevBasis& b, const EriOut& o, i
 // with the J[c,d] sums carried across the A chunks in registers, so J[c,d]
 // receives one atomic per element and quartet instead of one per A chunk.
 template <class PL, int CC, typename CT, bool FX>
-__device__ __forceinline__ void run_citem(const DevBasis& b, const EriOut& o, int P, int Qp, int pos,
-                                          const UnitRange& ur, bool active, const CT* __restrict__ tab, const RowAcc& acc, long long jb) {
+__device__ __forceinline__ void run_citem(ArgP ap, const Bra& br, int col, const UnitRange& ur, bool active,
+                                          const CT* __restrict__ tab, const RowAcc& acc) {
   using CK = Chunk<PL, CC>;  // A chunk 0: the C range of every A chunk of CC
   constexpr int ND = PL::ND, NCDL = (CK::c1 - CK::c0) * ND;
   double jcd[NCDL];
 #pragma unroll
   for (int c = 0; c < NCDL; ++c) jcd[c] = 0.0;
-  run_agroup<PL, CC, 0, CT, FX>(b, o, P, Qp, pos, ur, active, tab, acc, jcd, jb);
-  double* Jo = (o.mode == MODE_FOCK) ? o.F : o.J;
-  if (Jo && active && P != Qp && jb >= 0) {
-    const int lane = threadIdx.x & 63;
+  run_agroup<PL, CC, 0, CT, FX>(ap, br, col, ur, active, tab, acc, jcd);
+  ap = refetch(ap);
+  const unsigned lane = threadIdx.x & 63;
+  if (ap->den[0].J && active && br.posP != col + (int)lane) {
+    double* Jp = ap->den[0].Jpos + cl(ap->jblk, col >> 6) + 64LL * (CK::c0 * ND);
 #pragma unroll
-    for (int c = 0; c < NCDL; ++c) acc_add(o.Jpos + jb + 64LL * (CK::c0 * ND + c) + lane, jcd[c], FX);
-  } else if (Jo && active && P != Qp) {
-    const int A = uni(b.sp_A[P]), C = b.sp_A[Qp], Dsh = b.sp_B[Qp];
-    long long N, msh;
-    mol_layout(b, A, N, msh);
-    Jo = shifted(Jo, msh);
-    const int aoC = b.shell_ao[C] + CK::c0, aoD = b.shell_ao[Dsh];
-#pragma unroll
-    for (int c = 0; c < NCDL; ++c) acc_add(&Jo[(aoC + c / ND) * N + aoD + c % ND], jcd[c], FX);
+    for (int c = 0; c < NCDL; ++c) acc_add((double*)((ASUKA_GLOB char*)Jp + (8 * lane + 512 * c)), jcd[c], FX);
   }
 }
 
 // Wave item `item` of a unit: a C chunk with its A chunks for CARRY plans,
 // one chunk otherwise.
 template <class PL, int CC, typename CT, bool FX>
-__device__ __forceinline__ void dispatch_citem(int cc, const DevBasis& b, const EriOut& o, int P, int Qp, int pos,
-                                               const UnitRange& ur, bool active, const CT* __restrict__ tab, const RowAcc& acc,
-                                               long long jb) {
+__device__ __forceinline__ void dispatch_citem(int cc, ArgP ap, const Bra& br, int col, const UnitRange& ur,
+                                               bool active, const CT* __restrict__ tab, const RowAcc& acc) {
   if constexpr (!PL::CARRY) {
-    dispatch_chunk<PL, 0, CT, FX>(cc, b, o, P, Qp, pos, ur, active, tab, acc, jb);
+    dispatch_chunk<PL, 0, CT, FX>(cc, ap, br, col, ur, active, tab, acc);
   } else if constexpr (CC < PL::SPLIT_C) {
     if (cc == CC) {
-      run_citem<PL, CC, CT, FX>(b, o, P, Qp, pos, ur, active, tab, acc, jb);
+      run_citem<PL, CC, CT, FX>(ap, br, col, ur, active, tab, acc);
       return;
     }
-    dispatch_citem<PL, CC + 1, CT, FX>(cc, b, o, P, Qp, pos, ur, active, tab, acc, jb);
+    dispatch_citem<PL, CC + 1, CT, FX>(cc, ap, br, col, ur, active, tab, acc);
   }
 }
 
 // Work mapping: each workgroup pulls row tasks (wave units of one bra pair,
-// longest first) from the class pair's queue; its eight wavefronts take the task's
+// longest first) from the class pair's queue; its wavefronts take the task's
 // (unit, chunk) items in turn, so within a wave the bra pair and the chunk
 // (and with it all register indexing) are uniform. With LDS accumulators the
 // task's J[a,b] block and K rows of a and b are summed in LDS and added to
 // J/K once at the end of the task.
 //
-// Precision: CT is the kernel's arithmetic. Without o.mixed only the FP64
-// kernel runs and takes every unit. With o.mixed both run, each walking the
-// whole task list from its own queue head: a unit goes to the FP32 kernel when
-// every active quartet's bound Q_ab Q_cd max|D| is below tau (a wave-uniform
-// vote), else to the FP64 kernel, and the other kernel skips it. Separate
-// kernels keep the FP32 path's register allocation (and so its occupancy)
-// its own.
-//
-// The read-only inputs are also passed as __restrict__ arguments and rebound
-// into b, w and o: with no possible aliasing store (the J/K atomics) the
-// compiler can turn wave-uniform loads (wave unit, bra pair, bra primitive
-// pairs, D blocks of the bra) into scalar loads.
+// Precision: CT is the kernel's arithmetic. In mixed builds the FP64 and the
+// FP32 kernel each walk their own list of units (routed once per build);
+// without routed lists (vote) both walk all units, each from its own queue
+// head, and a unit goes to the FP32 kernel when every active quartet's bound
+// Q_ab Q_cd max|D| is below tau. Separate kernels keep the FP32 path's register
+// allocation (and so its occupancy) its own.
 // FX: accumulate in the 64-bit fixed point of deterministic builds
 // (EriOut::fixed), a separate instantiation so that the FP64-atomic kernels
 // carry none of its code or registers.
 template <class PL, typename CT, bool FX>
-__global__ __launch_bounds__(kGroupThreads) void eri_fast_kernel(DevBasis b, ClassWork w, EriOut o,
-                                                       const PrimPairF* __restrict__ ppf,
-                                                       const PrimPairF32* __restrict__ ppf32,
-                                                       const WaveUnit* __restrict__ units,
-                                                       const int* __restrict__ col_pair,
-                                                       const int* __restrict__ sp_A, const int* __restrict__ sp_B,
-                                                       const int* __restrict__ pp_start,
-                                                       const int* __restrict__ pp_count,
-                                                       const double* __restrict__ shell_xyz,
-                                                       const int* __restrict__ shell_ao,
-                                                       const double* __restrict__ Qb,
-                                                       const double* __restrict__ Dsp,
-                                                       const double* __restrict__ Dm) {
-  b.ppf = ppf;
-  b.ppf32 = ppf32;
-  b.sp_A = sp_A;
-  b.sp_B = sp_B;
-  b.pp_start = pp_start;
-  b.pp_count = pp_count;
-  b.shell_xyz = shell_xyz;
-  b.shell_ao = shell_ao;
-  b.Q = Qb;
-  b.Dsp = Dsp;
-  w.units = units;
-  w.col_pair = col_pair;
-  o.D = Dm;
+__global__ __launch_bounds__(kGroupThreads) void eri_fast_kernel(FastArgs args) {
+  (void)args;  // read through the kernel-argument segment, where it starts
+  ArgP ap = refetch((ArgP)__builtin_amdgcn_kernarg_segment_ptr());
   constexpr bool kF32 = sizeof(CT) == 4;
   constexpr int NIT = PL::CARRY ? PL::SPLIT_C : PL::NCH, NR = PL::NR;  // wave items per unit
   constexpr int NA = nc_(PL::la), NB = PL::NB;
@@ -737,7 +758,7 @@ __global__ __launch_bounds__(kGroupThreads) void eri_fast_kernel(DevBasis b, Cla
   constexpr int SCT = rys_c::lds_stride_of<CT>(NR);
   constexpr int TB = kLds ? rys_c::block_size_of<CT>(NR) : 1;
   constexpr int TBC = kLds ? rys_c::nint_of<CT>(NR) * SCT : 1;
-  const int wpg = w.wpg, nthr = 64 * w.wpg;  // the launch's block size (uniform)
+  const int wpg = ap->wpg, nthr = 64 * wpg;  // the launch's block size (uniform)
   __shared__ CT tct[TBC];
   const CT* gct;
   if constexpr (kF32)
@@ -750,12 +771,10 @@ __global__ __launch_bounds__(kGroupThreads) void eri_fast_kernel(DevBasis b, Cla
       tct[iv * SCT + f] = gct[t];
     }
   }
-  const bool use_acc = w.acc_colsC > 0;
-  const int nden = o.D2 ? 2 : 1;  // densities digested (accumulator sets in s_acc)
   RowAcc acc{};
   int nacc = 0;
-  if (use_acc) {  // row-task accumulators in s_acc, sized at launch
-    const int cC = w.acc_colsC, cD = w.acc_colsD;  // cD == 0: D columns share the C space
+  if (ap->acc_colsC > 0) {  // row-task accumulators in s_acc, sized at launch
+    const int cC = ap->acc_colsC, cD = ap->acc_colsD;  // cD == 0: D columns share the C space
     acc.on = true;
     acc.colsC = cC;
     acc.colsD = cD > 0 ? cD : cC;
@@ -766,154 +785,116 @@ __global__ __launch_bounds__(kGroupThreads) void eri_fast_kernel(DevBasis b, Cla
     acc.kbd = cD > 0 ? acc.kbc + NB * cC : acc.kbc;
     nacc = NA * NB + (NA + NB) * (cC + cD);
     acc.stride = nacc;
-    for (int t = threadIdx.x; t < nacc * nden; t += nthr) s_acc[t] = 0.0;
+    for (int t = threadIdx.x; t < nacc * ap->nden; t += nthr) s_acc[t] = 0.0;
   }
   __shared__ int s_task, s_work;
   if (threadIdx.x == 0) s_work = 0;
   __syncthreads();
   const CT* tab = kLds ? tct : gct;
-  const int lane = threadIdx.x & 63;
-
-  unsigned int* queue = kF32 ? w.queue32 : w.queue;
-  // launched with kGroupThreads-thread blocks; blockDim is not read because
-  // the compiler cannot prove it uniform, which would make the loops divergent
-  const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const unsigned lane = threadIdx.x & 63;
+  // blockDim is not read because the compiler cannot prove it uniform, which
+  // would make the loops divergent
+  const int wib = uni((int)(threadIdx.x >> 6));
   for (;;) {  // persistent workgroups pull row tasks from the class pair's queue
-    if (threadIdx.x == 0) s_task = (int)atomicAdd(queue, 1u);
+    ap = refetch(ap);
+    if (threadIdx.x == 0) s_task = (int)atomicAdd(ap->queue, 1u);
     __syncthreads();
-    const int t = s_task;
-    if (t >= w.ntasks) break;  // uniform per workgroup; every workgroup gets here
-    const RowTask tk = w.tasks[t];  // routed lists hold empty tasks (nu = 0): no unit to read
-    int P = 0;
-    if (tk.nu > 0) P = uni(w.units[tk.u0].P);
+    const int t = uni(s_task);
+    if (t >= ap->ntasks) break;  // uniform per workgroup; every workgroup gets here
+    const int u0 = cl((const int*)ap->tasks, 2LL * t), nu = cl((const int*)ap->tasks, 2LL * t + 1);
     bool worked = false;  // this wave digested an item of the task (uniform)
-    // a wave item is one chunk of a unit, or for CARRY plans one C chunk with
-    // its A chunks in sequence; items chunk-major: the waves of a workgroup
-    // run the same chunk's code
-    // over different units (a split plan's chunks are separate code regions,
-    // together far larger than the instruction cache)
-    for (int item = wib; item < tk.nu * NIT; item += wpg) {  // uniform per wave
-      const int chunk = item / tk.nu;
-      const int ui = item - chunk * tk.nu;
-      const WaveUnit un = w.units[tk.u0 + ui];
-      bool active = lane < (int)un.ncol;
-      // the lane's ket position: units start at 64-position block boundaries,
-      // so every lane's position (tail lanes: padding) is inside the lists
-      const int pos = un.col + lane;
-      const int Qp = w.col_pair[active ? pos : un.col];
-      double bound = 0.0;
-      if (active) {
-        bound = (b.Q[P] * b.kq[pos]) * fmax(b.Dsp[P], b.kd[pos]);
-        if (o.eps_density > 0.0) active = bound >= o.eps_density;
-      }
-      if (!wave_any(active)) continue;  // the whole unit is density-screened
-      if (!w.routed) {  // without routed lists each kernel takes the units its vote gives it
-        const bool lowp = o.mixed && wave_all(!active || bound < o.tau_mixed);
-        if (lowp != kF32) continue;  // the other precision's kernel takes this unit
-      }
-      worked = true;
-      // the unit's primitive pairs (see run_chunk)
-      UnitRange ur = unit_range(un, b.pp_count[P], false);
-      ur.i0 = uni(ur.i0), ur.ni = uni(ur.ni), ur.j0 = uni(ur.j0), ur.j1 = uni(ur.j1);
-      if (o.counters && chunk == 0) {
-        // statistics: one atomic per counter and wave; quartets are counted by
-        // their first slice
-        const bool first_slice = ur.i0 == 0 && ur.j0 == 0;
-        const int A = b.sp_A[P], B = b.sp_B[P], C = b.sp_A[Qp], Dsh = b.sp_B[Qp];
-        unsigned long long* cnt = o.counters + kCountStride * w.cp_index;
-        const unsigned long long kq =
-            active && first_slice ? (unsigned long long)b.pp_count0[P] * (unsigned long long)b.pp_count0[Qp] : 0ull;
-        const int bin = (((A != B) << 2) | ((C != Dsh) << 1) | (P != Qp));
-        for (int k = 0; k < 8; ++k) {
-          const unsigned long long m = __ballot(active && first_slice && bin == k);
-          if (m && lane == 0) atomicAdd(cnt + k, (unsigned long long)__popcll(m));
+    if (nu > 0) {         // routed lists hold empty tasks: no unit to read
+      Bra br;
+      br.P = cl((const int*)ap->units, 4LL * u0);
+      br.A = cl(ap->sp_A, br.P);
+      br.B = cl(ap->sp_B, br.P);
+      br.ab0 = cl(ap->pp_start, br.P);
+      br.posP = cl(ap->pos_of_sp, br.P);
+      br.aoA = cl(ap->shell_ao, br.A);
+      br.aoB = cl(ap->shell_ao, br.B);
+      const int mol = cl(ap->shell_mol, br.A);
+      br.N = cl(ap->mol_n, mol);
+      br.msh = cl(ap->mol_shift, mol);
+      // a wave item is one chunk of a unit, or for CARRY plans one C chunk with
+      // its A chunks in sequence; items chunk-major: the waves of a workgroup
+      // run the same chunk's code over different units (a split plan's chunks
+      // are separate code regions, together far larger than the instruction cache)
+      for (int item = wib; item < nu * NIT; item += wpg) {  // uniform per wave
+        ap = refetch(ap);
+        const int chunk = NIT == 1 ? 0 : item / nu;
+        const int ui = item - chunk * nu;
+        union {
+          u32x4 v;
+          WaveUnit u;
+        } un;
+        un.v = cl((const u32x4*)ap->units, u0 + ui);
+        const int col = un.u.col;
+        // the lane's ket position is col + lane: units start at 64-position
+        // block boundaries, so tail lanes read padding positions of the block
+        bool active = lane < (unsigned)un.u.ncol;
+        const double bound = (cl(ap->Q, br.P) * gl<double>(ap->kq + col, 8 * lane)) *
+                             fmax(cl(ap->Dsp, br.P), gl<double>(ap->kd + col, 8 * lane));
+        if (ap->eps_density > 0.0) active = active && bound >= ap->eps_density;
+        if (!wave_any(active)) continue;  // the whole unit is density-screened
+        if (ap->vote) {
+          const bool lowp = wave_all(!active || bound < ap->tau_mixed);
+          if (lowp != kF32) continue;  // the other precision's kernel takes this unit
         }
-        const unsigned long long ksum = (unsigned long long)wave_sum((double)kq);
-        const unsigned long long nact = (unsigned long long)__popcll(__ballot(active && first_slice));
-        // primitive quartets the loops evaluate (after the primitive-quartet
-        // cut) and the lane slots the wave spends on them (64 x the longest lane)
-        long long nev = 0;
-        if (active && ur.ni > 0) {
-          const int cd0 = b.pp_start[Qp], ncd = min(b.pp_count[Qp], ur.j1);
-          const double kcut = o.eps_prim > 0.0 ? o.eps_prim / b.ppf[b.pp_start[P] + ur.i0].q : 0.0;
-          int j = ur.j0;
-          while (j < ncd && !(b.ppf[cd0 + j].q < kcut)) ++j;
-          nev = (long long)ur.ni * (j - ur.j0);
-        }
-        const double nevs = wave_sum((double)nev);
-        double nmax = (double)nev;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) nmax = fmax(nmax, __shfl_xor(nmax, off));
-        if (lane == 0) {
-          atomicAdd(cnt + 8, ksum);
-          atomicAdd(cnt + 11, (unsigned long long)nevs);
-          atomicAdd(cnt + 12, 64ull * (unsigned long long)nmax);
-          if (kF32) {
-            atomicAdd(cnt + 9, nact);
-            atomicAdd(cnt + 10, ksum);
-          }
-        }
+        worked = true;
+        // inactive lanes (tail, screened) run with an empty primitive loop and no
+        // atomics so the wave stays converged for the cross-lane reductions
+        const UnitRange ur = unit_range(un.u, cl(ap->pp_count, br.P), false);
+        dispatch_citem<PL, 0, CT, FX>(chunk, ap, br, col, ur, active, tab, acc);
       }
-      // inactive lanes (tail, screened) run with an empty primitive loop and no
-      // atomics so the wave stays converged for the cross-lane reductions
-      // the unit's block of the ket-position buffers (units start at block boundaries)
-      const long long jb = o.jblk ? o.jblk[un.col >> 6] : -1LL;
-      dispatch_citem<PL, 0, CT, FX>(chunk, b, o, P, Qp, pos, ur, active, tab, acc, jb);
-    }
-    if (use_acc) {
-      if (worked && lane == 0) s_work = 1;
-      __syncthreads();  // the task's contributions are in LDS
-      if (s_work) {
-        const int A = b.sp_A[P], B = b.sp_B[P];
-        long long N, msh;
-        mol_layout(b, A, N, msh);
-        const long long aoA = b.shell_ao[A], aoB = b.shell_ao[B];
-        const int cC = w.acc_colsC, cD = w.acc_colsD;
-        const int* mlao = b.mol_lao + b.shell_mol[A] * (ASUKA_LMAX + 1);  // the molecule's AO lists
-        const int* laoC = b.lao_ao + w.lao_offC + mlao[PL::lc];
-        const int* laoD = b.lao_ao + (cD > 0 ? w.lao_offD + mlao[PL::ld] : w.lao_offC + mlao[PL::lc]);
-        const int cDe = cD > 0 ? cD : cC;
-        // compact columns of the C and D lists (EriOut::Kc)
-        const int gC = w.lao_offC + mlao[PL::lc], gD = cD > 0 ? w.lao_offD + mlao[PL::ld] : gC;
-        for (int t2 = threadIdx.x; t2 < nacc * nden; t2 += nthr) {
-          const double v = s_acc[t2];  // fixed builds: the bits of an integer sum
-          if (__double_as_longlong(v) == 0LL) continue;
-          s_acc[t2] = 0.0;
-          const bool second = t2 >= nacc;
-          double* Jo = shifted(second ? o.J2 : ((o.mode == MODE_FOCK) ? o.F : o.J), msh);
-          double* Ko = shifted(second ? o.K2 : ((o.mode == MODE_FOCK) ? o.F : o.K), msh);
-          double* Kc = second ? o.Kc2 : o.Kc;  // uniform
-          int r = second ? t2 - nacc : t2;
-          if (r < NA * NB) {
-            acc_add_sum(&Jo[(aoA + r / NB) * N + aoB + r % NB], v, FX);
-            continue;
-          }
-          r -= NA * NB;
-          long long row, k;  // the K row (AO) and the entry's index in its column list
-          int g;             // first compact column of that list
-          const int* lao;
-          if (r < NA * cC) {
-            row = aoA + r / cC, k = r % cC, g = gC, lao = laoC;
-          } else if ((r -= NA * cC), cD > 0 && r < NA * cD) {
-            row = aoA + r / cD, k = r % cD, g = gD, lao = laoD;
-          } else {
-            if (cD > 0) r -= NA * cD;
-            if (r < NB * cC) {
-              row = aoB + r / cC, k = r % cC, g = gC, lao = laoC;
-            } else {
-              r -= NB * cC;
-              row = aoB + r / cDe, k = r % cDe, g = gD, lao = laoD;
+      if (acc.on) {
+        if (worked && lane == 0) s_work = 1;
+        __syncthreads();  // the task's contributions are in LDS
+        ap = refetch(ap);
+        if (s_work) {
+          const long long N = br.N, msh = br.msh, aoA = br.aoA, aoB = br.aoB;
+          const int cC = ap->acc_colsC, cD = ap->acc_colsD, nden = ap->nden;
+          const int* mlao = ap->mol_lao + mol * (ASUKA_LMAX + 1);  // the molecule's AO lists
+          // compact columns of the C and D lists (EriOut::Kc)
+          const int gC = ap->lao_offC + mlao[PL::lc], gD = cD > 0 ? ap->lao_offD + mlao[PL::ld] : gC;
+          const int* lao_ao = ap->lao_ao;
+          const int cDe = cD > 0 ? cD : cC;
+          for (int t2 = threadIdx.x; t2 < nacc * nden; t2 += nthr) {
+            const double v = s_acc[t2];  // fixed builds: the bits of an integer sum
+            if (__double_as_longlong(v) == 0LL) continue;
+            s_acc[t2] = 0.0;
+            const bool second = t2 >= nacc;
+            const ASUKA_CONST FastDen* dn = &ap->den[second ? 1 : 0];
+            int r = second ? t2 - nacc : t2;
+            if (r < NA * NB) {
+              acc_add_sum(dn->J + msh + (aoA + r / NB) * N + aoB + r % NB, v, FX);
+              continue;
             }
+            r -= NA * NB;
+            long long row, k;  // the K row (AO) and the entry's index in its column list
+            int g;             // first compact column of that list
+            if (r < NA * cC) {
+              row = aoA + r / cC, k = r % cC, g = gC;
+            } else if ((r -= NA * cC), cD > 0 && r < NA * cD) {
+              row = aoA + r / cD, k = r % cD, g = gD;
+            } else {
+              if (cD > 0) r -= NA * cD;
+              if (r < NB * cC) {
+                row = aoB + r / cC, k = r % cC, g = gC;
+              } else {
+                r -= NB * cC;
+                row = aoB + r / cDe, k = r % cDe, g = gD;
+              }
+            }
+            if (dn->Kc)  // consecutive entries, consecutive addresses
+              acc_add_sum(dn->Kc + row * N + g + k, v, FX);
+            else
+              acc_add_sum(dn->K + msh + row * N + lao_ao[g + k], v, FX);
           }
-          if (Kc)  // consecutive entries, consecutive addresses
-            acc_add_sum(&Kc[row * N + g + k], v, FX);
-          else
-            acc_add_sum(&Ko[row * N + lao[k]], v, FX);
         }
       }
     }
     __syncthreads();  // accumulators are zero again; s_task and s_work may be overwritten
-    if (use_acc && threadIdx.x == 0) s_work = 0;
+    if (acc.on && threadIdx.x == 0) s_work = 0;
   }
 }
 
@@ -941,6 +922,35 @@ struct F32PlanOf {
   using type = Plan<PL::la, PL::lb, PL::lc, PL::ld, SA, SC>;
 };
 
+// The kernel arguments of a class pair's launch in one precision; false units
+// and tasks are w's (FP64 list) or, f32, the routed FP32 list.
+inline FastArgs fast_args(const DevBasis& b, const ClassWork& w, const EriOut& o, bool f32) {
+  FastArgs a{};
+  a.units = f32 && w.routed ? w.units32 : w.units;
+  a.tasks = f32 && w.routed ? w.tasks32 : w.tasks;
+  a.queue = f32 ? w.queue32 : w.queue;
+  a.pp = f32 ? (const void*)b.ppf32 : (const void*)b.ppf;
+  a.kpd = f32 ? b.kp32d : b.kp64;
+  a.kpf = b.kp32f;
+  a.kpoff = b.kpoff;
+  a.sp_A = b.sp_A, a.sp_B = b.sp_B, a.pp_start = b.pp_start, a.pp_count = b.pp_count;
+  a.shell_ao = b.shell_ao, a.shell_mol = b.shell_mol, a.mol_n = b.mol_n, a.mol_lao = b.mol_lao;
+  a.lao_ao = b.lao_ao, a.pos_of_sp = b.pos_of_sp, a.mol_shift = b.mol_shift, a.jblk = o.jblk;
+  a.shell_xyz = b.shell_xyz, a.Q = b.Q, a.Dsp = b.Dsp, a.kq = b.kq, a.kd = b.kd, a.kcd = b.kcd;
+  a.kpp = b.kpp, a.kao = b.kao, a.klao = b.klao;
+  const bool fock = o.mode == MODE_FOCK;
+  a.den[0] = FastDen{o.D, fock ? o.F : o.J, fock ? o.F : o.K, o.Dpos, o.Jpos, o.Kc};
+  a.den[1] = FastDen{o.D2, o.J2, o.K2, o.Dpos2, o.Jpos2, o.Kc2};
+  a.eps_density = o.eps_density, a.eps_prim = o.eps_prim, a.tau_mixed = o.tau_mixed;
+  a.ks = fock ? -0.5 : 1.0;
+  a.nden = o.D2 ? 2 : 1;
+  a.ntasks = (int)w.ntasks;
+  a.wpg = w.wpg;
+  a.vote = o.mixed && !w.routed;
+  a.acc_colsC = w.acc_colsC, a.acc_colsD = w.acc_colsD, a.lao_offC = w.lao_offC, a.lao_offD = w.lao_offD;
+  return a;
+}
+
 template <class PL, typename CT, bool FX = false>
 hipError_t launch_one(const DevBasis& b, const ClassWork& w, const EriOut& o, size_t lds, long long g, hipStream_t s) {
   if (lds > 64 * 1024) {
@@ -948,9 +958,8 @@ hipError_t launch_one(const DevBasis& b, const ClassWork& w, const EriOut& o, si
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL((eri_fast_kernel<PL, CT, FX>), dim3((unsigned)g), dim3(64 * w.wpg), lds, s, b, w, o, b.ppf, b.ppf32,
-                     w.units, w.col_pair, b.sp_A, b.sp_B, b.pp_start, b.pp_count, b.shell_xyz, b.shell_ao, b.Q,
-                     b.Dsp, o.D);
+  hipLaunchKernelGGL((eri_fast_kernel<PL, CT, FX>), dim3((unsigned)g), dim3(64 * w.wpg), lds, s,
+                     fast_args(b, w, o, sizeof(CT) == 4));
   return hipGetLastError();
 }
 
@@ -968,12 +977,7 @@ hipError_t launch_plan(const DevBasis& b, const ClassWork& w, const EriOut& o, h
   if (o.fixed) return launch_one<PL, double, true>(b, w, o, lds, g, s);
   hipError_t e = launch_one<PL, double>(b, w, o, lds, g, s);
   if (e != hipSuccess || !o.mixed) return e;
-  ClassWork w32 = w;
-  if (w.routed) {
-    w32.units = w.units32;
-    w32.tasks = w.tasks32;
-  }
-  return launch_one<typename F32PlanOf<PL>::type, float>(b, w32, o, lds, g, s);
+  return launch_one<typename F32PlanOf<PL>::type, float>(b, w, o, lds, g, s);
 }
 
 using Launcher = hipError_t (*)(const DevBasis&, const ClassWork&, const EriOut&, hipStream_t);

@@ -193,28 +193,17 @@ __device__ __forceinline__ void deriv_unit(const DevBasis& b, const GradFastArgs
   double gA[3] = {0, 0, 0}, gB[3] = {0, 0, 0}, gC[3] = {0, 0, 0};
   const int ab0 = uni_g(b.pp_start[P]) + ur.i0, nab = ur.ni;  // the unit's bra primitive pairs
   const int ncd = active ? min(b.kpp[pos].y, ur.j1) : 0;
-  // the lane's ket primitive pairs from the transposed tables (slots
-  // ks0 + 64 j, field f at kp64[f * kslots + slot]): one contiguous load
-  // per field across the wave (no prefetch of the next pair: its registers
-  // cost these kernels an occupancy step)
-  const int ks0 = (int)b.kpoff[uni_g(pos >> 6)] * 64 + (pos & 63);
-  const double* kt = b.kp64;
-  const long long ns = b.kslots;
-  auto ket = [&](int t, double* y) {
-    y[0] = kt[t];           // eta
-    y[1] = (kt + ns)[t];     // 1/eta
-    y[2] = (kt + 2 * ns)[t]; // ck
-    y[3] = (kt + 3 * ns)[t]; // P
-    y[4] = (kt + 4 * ns)[t];
-    y[5] = (kt + 5 * ns)[t];
-    y[6] = (kt + 6 * ns)[t]; // P - C
-    y[7] = (kt + 7 * ns)[t];
-    y[8] = (kt + 8 * ns)[t];
-    y[9] = (kt + 10 * ns)[t]; // exponent of the C primitive
-  };
+  // the lane's ket primitive pairs from the transposed tables
+  // (DevBasis::kpoff): one contiguous load per field across the wave (no
+  // prefetch of the next pair: its registers cost these kernels an occupancy
+  // step)
+  const double* kt = b.kp64 + b.kpoff[uni_g(pos >> 6)] * (64 * kKet64) + (pos & 63);
   for (int j = ur.j0; j < ncd; ++j) {
     double y[10];
-    ket(ks0 + 64 * j, y);
+    const double* kj = kt + (long long)j * (64 * kKet64);
+#pragma unroll
+    for (int f = 0; f < 9; ++f) y[f] = kj[64 * f];  // eta, 1/eta, ck, P, P - C
+    y[9] = kj[64 * 10];                             // exponent of the C primitive
     const double q = y[0], iq = y[1], ckq = y[2], c2 = 2.0 * y[9];
     const double Yp[3] = {y[3], y[4], y[5]};
     const double QC[3] = {y[6], y[7], y[8]};

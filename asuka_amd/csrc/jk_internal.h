@@ -58,6 +58,9 @@ enum EriMode : int {
   MODE_SCHWARZ = 3,  // Q[P] = sqrt(max diag (P|P))
 };
 
+// Fields of a slot row of the transposed ket tables (DevBasis::kpoff).
+constexpr int kKet64 = 11, kKet32d = 3, kKet32f = 7;
+
 // Device-side view of a context (passed by value to kernels).
 struct DevBasis {
   const double* shell_xyz;   // (nshell, 3)
@@ -92,17 +95,18 @@ struct DevBasis {
   const double* kcd;
   // The ket primitive pairs by position, transposed so that the lanes of a
   // wave read the j-th primitive pair of their kets at consecutive addresses:
-  // block k's primitive j of lane l is slot (kpoff[k] + j) * 64 + l, field f
-  // of slot t at kp64[f * kslots + t] (PrimPairF's ten fields in order, then
-  // the exponent of the pair's first primitive (PrimPair::a_exp, for the
+  // block k's primitive j is slot row kpoff[k] + j, and field f of lane l of
+  // row s is kp64[(s * kKet64 + f) * 64 + l] (PrimPairF's ten fields in order,
+  // then the exponent of the pair's first primitive (PrimPair::a_exp, for the
   // derivative kernels); FP64 kernels) and, for the FP32 kernels,
-  // kp32d[f * kslots + t] (Px, Py, Pz) and kp32f[f * kslots + t] (eta,
-  // inv_eta, ck, PAx, PAy, PAz, q).
+  // kp32d[(s * kKet32d + f) * 64 + l] (Px, Py, Pz) and kp32f[(s * kKet32f + f)
+  // * 64 + l] (eta, inv_eta, ck, PAx, PAy, PAz, q): one base a row, the fields
+  // at fixed offsets from it.
   const long long* kpoff;
   const double* kp64;
   const double* kp32d;
   const float* kp32f;
-  long long kslots;
+  const int* pos_of_sp;  // ket position of each shell pair (-1: none)
   int nao;
   int nsp;
 };
