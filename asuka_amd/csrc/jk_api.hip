@@ -104,6 +104,7 @@ struct ClassPairHost {
   long long ntasks0 = 0;
   std::vector<std::pair<int, std::pair<RowTask*, long long>>> cuts;  // other cuts made so far
   double tuned_ms = 0.0;                  // time of the class pair's launch when tuned (0: not tuned)
+  bool route = false;                     // mixed builds route its units to an FP64 and an FP32 launch
   long long rtask_off = 0;                // first of its remapped row tasks (routed mixed builds)
 };
 
@@ -123,6 +124,19 @@ struct ClassPairHost {
 // -> 2.41 ms.
 static constexpr long long kSliceWaves = 8192;
 static inline long long slice_min(int nroots) { return std::max(2, 48 / (nroots * nroots)); }
+
+// Mixed builds split the units of a class pair into an FP64 and an FP32 launch
+// when it has more wave items than this (16 a SIMD); smaller class pairs run
+// all of them in FP64, in one launch: both launches would take as long as
+// their longest item. A caller that sets the FP32 cut itself (opts.tau_mixed >
+// 0) gets every class pair split. Measured, all split / above 4096 / 16384 /
+// 65536 / none: (H2O)3 cc-pVDZ Fock build 1214 / 938 / 823 / 821 / 821 us,
+// (H2O)5 two densities 2033 / 1983 / 1816 / 1783 / 1782, (H2O)14 11200 / 11180
+// / 11241 / 11479 / 12289, (H2O)8 cc-pVTZ 48.3 / 48.2 / 48.3 / 50.9 / 53.0 ms.
+// The largest class pair is split from kRouteMinLargest on, so that a mixed
+// build does run FP32 kernels from two molecules on (+40 us at (H2O)3).
+static constexpr long long kRouteMin = 16384;
+static constexpr long long kRouteMinLargest = 2048;
 
 // blk_k: largest primitive-pair count of each 64-position ket block.
 static void slice_units(const std::vector<int>& blk_k, ClassPairHost& cp, std::vector<WaveUnit>& units) {
@@ -379,56 +393,59 @@ __global__ void k_pos_dmax(const int* __restrict__ col, const double* __restrict
 // its quartets' bounds Q_ab Q_cd max(D_ab, D_cd): (Q_ab Q_first) max(D_ab,
 // max D_cd) with Q_first the unit's largest ket bound (its first position; ket
 // lists are Q-descending) and max D_cd the running block max at its last
-// position. f32[u] = 1 when that bound is below tau (every quartet of the
-// unit is then below tau: the FP32 kernel's share), f64[u] = 1 otherwise;
-// both 0 when it is below eps_density (every quartet density-screened). A
+// position. flags[u] = 2^32 when that bound is below tau (every quartet of the
+// unit is then below tau: the FP32 kernel's share), 1 otherwise, 0 when it is
+// below eps_density (every quartet density-screened): one sum counts both. A
 // unit kept by the bound whose quartets are all screened is skipped in the
 // kernel, which tests each quartet itself.
 __global__ void k_route_units(DevBasis b, const WaveUnit* __restrict__ units, const double* __restrict__ qcol,
                               const double* __restrict__ dmaxcol, long long nunits, double eps_density, double tau,
-                              int* f64, int* f32) {
+                              unsigned long long* flags) {
   for (long long u = blockIdx.x * (long long)blockDim.x + threadIdx.x; u < nunits;
        u += (long long)gridDim.x * blockDim.x) {
     const WaveUnit un = units[u];
     const double hi = (b.Q[un.P] * qcol[un.col]) * fmax(b.Dsp[un.P], dmaxcol[un.col + un.ncol - 1]);
     const bool any = un.ncol > 0 && (eps_density > 0.0 ? hi >= eps_density : true);
-    const bool lowp = hi < tau;
-    f32[u] = (any && lowp) ? 1 : 0;
-    f64[u] = (any && !lowp) ? 1 : 0;
+    flags[u] = !any ? 0ull : hi < tau ? 1ull << 32 : 1ull;
   }
 }
 
 // The routed units, in their original order, into the FP64 and FP32 lists
-// (pos: exclusive sums of the flags).
-__global__ void k_scatter_units(const WaveUnit* __restrict__ units, long long nunits, const int* __restrict__ f64,
-                                const int* __restrict__ f32, const int* __restrict__ pos64,
-                                const int* __restrict__ pos32, WaveUnit* u64, WaveUnit* u32) {
+// (pos: exclusive sums of the flags, FP64 in the low and FP32 in the high half).
+__global__ void k_scatter_units(const WaveUnit* __restrict__ units, long long nunits,
+                                const unsigned long long* __restrict__ flags,
+                                const unsigned long long* __restrict__ pos, WaveUnit* u64, WaveUnit* u32) {
   for (long long u = blockIdx.x * (long long)blockDim.x + threadIdx.x; u < nunits; u += (long long)gridDim.x * blockDim.x) {
-    if (f32[u]) u32[pos32[u]] = units[u];
-    if (f64[u]) u64[pos64[u]] = units[u];
+    const unsigned long long f = flags[u], p = pos[u];
+    if (f >> 32) u32[p >> 32] = units[u];
+    if (f & 1ull) u64[p & 0xffffffffull] = units[u];
   }
 }
 
-// A class pair's row tasks (units [ubase + u0, ubase + u0 + nu) of the full
-// list) as the ranges their units occupy in the two routed lists; a range may
-// be empty.
-__global__ void k_route_tasks(const RowTask* __restrict__ tasks, long long ntasks, long long ubase,
-                              const int* __restrict__ pos64, const int* __restrict__ pos32, RowTask* t64,
-                              RowTask* t32) {
+// Row tasks (units [u0, u0 + nu) of the full list, every routed class pair's)
+// as the ranges their units occupy in the two routed lists; a range may be empty.
+__global__ void k_route_tasks(const RowTask* __restrict__ tasks, long long ntasks,
+                              const unsigned long long* __restrict__ pos, RowTask* t64, RowTask* t32) {
   for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < ntasks; t += (long long)gridDim.x * blockDim.x) {
     const RowTask tk = tasks[t];
-    const long long g0 = ubase + tk.u0, g1 = g0 + tk.nu;
-    t64[t] = RowTask{pos64[g0], pos64[g1] - pos64[g0]};
-    t32[t] = RowTask{pos32[g0], pos32[g1] - pos32[g0]};
+    const unsigned long long p0 = pos[tk.u0], p1 = pos[(long long)tk.u0 + tk.nu];
+    t64[t] = RowTask{(int)(p0 & 0xffffffffull), (int)((p1 & 0xffffffffull) - (p0 & 0xffffffffull))};
+    t32[t] = RowTask{(int)(p0 >> 32), (int)((p1 >> 32) - (p0 >> 32))};
   }
+}
+
+// A class pair's row tasks with its first unit added (its units' places in the full list).
+__global__ void k_shift_tasks(const RowTask* __restrict__ tasks, long long ntasks, int ubase, RowTask* out) {
+  for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < ntasks; t += (long long)gridDim.x * blockDim.x)
+    out[t] = RowTask{tasks[t].u0 + ubase, tasks[t].nu};
 }
 
 // Counters (EriOut::counters) of a class pair of the register kernels, one
 // wavefront per wave unit: what those kernels evaluate follows from the
-// screening alone, so they carry no counting code. f32: the units' precision
-// in mixed builds (null: all FP64).
+// screening alone, so they carry no counting code. flags: the units' routing
+// (k_route_units; null: all FP64).
 __global__ __launch_bounds__(256) void k_count_units(const DevBasis b, const WaveUnit* __restrict__ units,
-                                                     long long nunits, const int* __restrict__ f32,
+                                                     long long nunits, const unsigned long long* __restrict__ flags,
                                                      const int* __restrict__ col_pair, double eps_density,
                                                      double eps_prim, unsigned long long* cnt) {
   const int lane = threadIdx.x & 63;
@@ -466,7 +483,7 @@ __global__ __launch_bounds__(256) void k_count_units(const DevBasis b, const Wav
       atomicAdd(cnt + 8, ksum);
       atomicAdd(cnt + 11, (unsigned long long)nevs);
       atomicAdd(cnt + 12, 64ull * (unsigned long long)nmax);
-      if (f32 && f32[k]) {
+      if (flags && (flags[k] >> 32)) {
         atomicAdd(cnt + 9, nact);
         atomicAdd(cnt + 10, ksum);
       }
@@ -533,7 +550,7 @@ struct asuka_jk_ctx {
   // entries, the last 0), their exclusive sums, the two routed unit lists, the
   // remapped row tasks of every class pair (rtask_cap entries each) and the
   // scan scratch
-  int *d_rf64 = nullptr, *d_rf32 = nullptr, *d_rp64 = nullptr, *d_rp32 = nullptr;
+  unsigned long long *d_rflag = nullptr, *d_rpos = nullptr;
   // per ket position: Q of the pair (0 for padding) and, per build, the
   // running max of the pairs' max|D| from the position's 64-block start
   double *d_qcol = nullptr, *d_dmaxcol = nullptr;
@@ -541,7 +558,8 @@ struct asuka_jk_ctx {
   int* d_pos_of_sp = nullptr;      // position of each shell pair in the ket lists (-1: none)
   std::vector<int> h_shell_lao;    // host copy of DevBasis::shell_lao
   WaveUnit *d_units64 = nullptr, *d_units32 = nullptr;
-  RowTask *d_rtasks64 = nullptr, *d_rtasks32 = nullptr;
+  RowTask *d_rtasks = nullptr, *d_rtasks64 = nullptr, *d_rtasks32 = nullptr;  // all routed class pairs' row tasks
+  long long nrtasks = 0;
   long long rtask_cap = 0;
   void* d_scan_tmp = nullptr;
   size_t scan_tmp_bytes = 0;
@@ -623,26 +641,35 @@ static bool row_acc_fits(const asuka_jk_ctx* ctx, int la, int lb, int lc, int ld
   return bytes <= std::min(ctx->row_acc_max, ctx->lds_per_group - root_table_lds(nr) - 1024);
 }
 
-// Offsets of each class pair's remapped row tasks (of its current cut) in the
-// routed task arrays, which grow when a cut needs more room (context creation
-// and the autotuner's re-cuts; never during a build).
-static int route_task_layout(asuka_jk_ctx* ctx) {
+// The routed class pairs' row tasks (of their current cuts) end to end, with
+// the room their remapped copies take, which grows when a cut needs more
+// (context creation and the autotuner's re-cuts; never during a build).
+static int route_task_layout(asuka_jk_ctx* ctx, hipStream_t s) {
   long long tot = 0;
   for (auto& cp : ctx->cps) {
     cp.rtask_off = tot;
-    tot += cp.ntasks;
+    if (cp.route) tot += cp.ntasks;
   }
-  tot = std::max<long long>(1, tot);
-  if (tot > ctx->rtask_cap) {
-    RowTask *a = nullptr, *b = nullptr;
-    HIP_CHECK(hipMalloc(&a, sizeof(RowTask) * (size_t)tot));
-    ctx->owned.push_back(a);
-    HIP_CHECK(hipMalloc(&b, sizeof(RowTask) * (size_t)tot));
-    ctx->owned.push_back(b);
-    ctx->d_rtasks64 = a;
-    ctx->d_rtasks32 = b;
-    ctx->rtask_cap = tot;
+  ctx->nrtasks = tot;
+  const long long cap = std::max<long long>(1, tot);
+  if (cap > ctx->rtask_cap) {
+    for (RowTask** p : {&ctx->d_rtasks, &ctx->d_rtasks64, &ctx->d_rtasks32}) {
+      RowTask* a = nullptr;
+      HIP_CHECK(hipMalloc(&a, sizeof(RowTask) * (size_t)cap));
+      ctx->owned.push_back(a);
+      *p = a;
+    }
+    ctx->rtask_cap = cap;
   }
+  for (auto& cp : ctx->cps) {
+    if (!cp.route || cp.ntasks <= 0) continue;
+    const RowTask* t = cp.d_tasks_own ? cp.d_tasks_own : ctx->d_tasks + cp.task_start;
+    const long long g = std::min<long long>((cp.ntasks + 255) / 256, 65535);
+    hipLaunchKernelGGL(k_shift_tasks, dim3((unsigned)g), dim3(256), 0, s, t, cp.ntasks, (int)cp.unit_start,
+                       ctx->d_rtasks + cp.rtask_off);
+  }
+  HIP_CHECK(hipGetLastError());
+  HIP_CHECK(hipStreamSynchronize(s));
   return ASUKA_OK;
 }
 
@@ -749,11 +776,13 @@ static int pos_layout(asuka_jk_ctx* ctx, const std::vector<int>& col) {
   return ASUKA_OK;
 }
 
-static int route_alloc(asuka_jk_ctx* ctx) {
+static int route_alloc(asuka_jk_ctx* ctx, hipStream_t s) {
+  bool any = false;
+  for (const auto& cp : ctx->cps) any = any || cp.route;
+  if (!any) return ASUKA_OK;  // mixed builds run every class pair in FP64
   const long long n = (long long)ctx->h_units.size();
-  const size_t ni = sizeof(int) * (size_t)(n + 1);
-  int** flags[4] = {&ctx->d_rf64, &ctx->d_rf32, &ctx->d_rp64, &ctx->d_rp32};
-  for (int** f : flags) {
+  const size_t ni = sizeof(unsigned long long) * (size_t)(n + 1);
+  for (unsigned long long** f : {&ctx->d_rflag, &ctx->d_rpos}) {
     HIP_CHECK(hipMalloc((void**)f, ni));
     ctx->owned.push_back(*f);
     HIP_CHECK(hipMemset(*f, 0, ni));  // context creation, not a build: the flags' last entry stays 0
@@ -763,11 +792,11 @@ static int route_alloc(asuka_jk_ctx* ctx) {
   ctx->owned.push_back(ctx->d_units64);
   HIP_CHECK(hipMalloc((void**)&ctx->d_units32, nu));
   ctx->owned.push_back(ctx->d_units32);
-  HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, ctx->scan_tmp_bytes, ctx->d_rf64, ctx->d_rp64, (int)(n + 1)));
+  HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, ctx->scan_tmp_bytes, ctx->d_rflag, ctx->d_rpos, (int)(n + 1)));
   ctx->scan_tmp_bytes = std::max<size_t>(ctx->scan_tmp_bytes, 256);
   HIP_CHECK(hipMalloc(&ctx->d_scan_tmp, ctx->scan_tmp_bytes));
   ctx->owned.push_back(ctx->d_scan_tmp);
-  return route_task_layout(ctx);
+  return route_task_layout(ctx, s);
 }
 
 extern "C" {
@@ -1422,6 +1451,15 @@ static int ctx_build(const asuka_basis_desc* bd, const std::vector<int>* shell_m
       ctx->ntasks += cp.nquartets;
     }
   }
+  {  // class pairs that mixed builds split (kRouteMin)
+    auto items = [](const ClassPairHost& c) { return c.nunits * eri_fast_nch(c.la, c.lb, c.lc, c.ld); };
+    ClassPairHost* big = nullptr;
+    for (auto& cp : ctx->cps) {
+      cp.route = items(cp) > (opts->tau_mixed > 0.0 ? 0 : kRouteMin);
+      if (!big || items(cp) > items(*big)) big = &cp;
+    }
+    if (big && items(*big) > kRouteMinLargest) big->route = true;
+  }
   assign_streams(ctx);
   col_all.resize((col_all.size() + 63) / 64 * 64, -1);
   if ((rc = pos_layout(ctx, col_all))) return rc;
@@ -1440,7 +1478,7 @@ static int ctx_build(const asuka_basis_desc* bd, const std::vector<int>* shell_m
     std::vector<unsigned int> qz(2 * std::max<size_t>(1, ctx->cps.size()), 0u);
     if ((rc = dev_upload(&ctx->d_queue, qz, own, s))) return rc;
   }
-  if ((rc = route_alloc(ctx))) return rc;
+  if ((rc = route_alloc(ctx, s))) return rc;
   HIP_CHECK(hipStreamSynchronize(s));
   *out = guard.release();
   return ASUKA_OK;
@@ -1666,20 +1704,20 @@ static int run_classes(asuka_jk_ctx* ctx, const EriOut& o, hipStream_t s, bool t
   // launches, and the units split (in order) into an FP64 and an FP32 list, so
   // each kernel of a class pair walks only its own units.
   const long long nu_all = (long long)ctx->h_units.size();
-  const bool routed = o.mixed && ctx->d_rf64 && nu_all > 0;
+  const bool routed = o.mixed && ctx->d_rflag && nu_all > 0;
   if (routed) {
     hipLaunchKernelGGL(k_pos_dmax, dim3((unsigned)ctx->nblk), dim3(64), 0, s, ctx->d_col_pair, dev->Dsp,
                        ctx->d_dmaxcol);
     HIP_CHECK(hipGetLastError());
     hipLaunchKernelGGL(k_route_units, dim3(grid_for(nu_all, 256)), dim3(256), 0, s, *dev, ctx->d_units, ctx->d_qcol,
-                       ctx->d_dmaxcol, nu_all, o.eps_density, o.tau_mixed, ctx->d_rf64, ctx->d_rf32);
+                       ctx->d_dmaxcol, nu_all, o.eps_density, o.tau_mixed, ctx->d_rflag);
     HIP_CHECK(hipGetLastError());
     size_t tb = ctx->scan_tmp_bytes;
-    HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(ctx->d_scan_tmp, tb, ctx->d_rf64, ctx->d_rp64, (int)(nu_all + 1), s));
-    tb = ctx->scan_tmp_bytes;
-    HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(ctx->d_scan_tmp, tb, ctx->d_rf32, ctx->d_rp32, (int)(nu_all + 1), s));
+    HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(ctx->d_scan_tmp, tb, ctx->d_rflag, ctx->d_rpos, (int)(nu_all + 1), s));
     hipLaunchKernelGGL(k_scatter_units, dim3(grid_for(nu_all, 256)), dim3(256), 0, s, ctx->d_units, nu_all,
-                       ctx->d_rf64, ctx->d_rf32, ctx->d_rp64, ctx->d_rp32, ctx->d_units64, ctx->d_units32);
+                       ctx->d_rflag, ctx->d_rpos, ctx->d_units64, ctx->d_units32);
+    hipLaunchKernelGGL(k_route_tasks, dim3(grid_for(ctx->nrtasks, 256)), dim3(256), 0, s, ctx->d_rtasks, ctx->nrtasks,
+                       ctx->d_rpos, ctx->d_rtasks64, ctx->d_rtasks32);
     HIP_CHECK(hipGetLastError());
   }
   // J[c,d] and D[c,d] by ket position for the register kernels of J/K and
@@ -1721,17 +1759,13 @@ static int run_classes(asuka_jk_ctx* ctx, const EriOut& o, hipStream_t s, bool t
     ClassWork w = work_of(ctx, cph, i);
     w.queue = queue + i;
     w.queue32 = queue + ncp + i;
-    if (routed && w.ntasks > 0 && eri_fast_has_plan(w.la, w.lb, w.lc, w.ld)) {
-      RowTask* t64 = ctx->d_rtasks64 + cph.rtask_off;
-      RowTask* t32 = ctx->d_rtasks32 + cph.rtask_off;
-      hipLaunchKernelGGL(k_route_tasks, dim3(grid_for(w.ntasks, 256)), dim3(256), 0, ls, w.tasks, w.ntasks,
-                         cph.unit_start, ctx->d_rp64, ctx->d_rp32, t64, t32);
-      HIP_CHECK(hipGetLastError());
+    oo.mixed = routed && cph.route ? 1 : 0;  // the other class pairs run in FP64
+    if (oo.mixed) {
       w.routed = 1;
       w.units = ctx->d_units64;
-      w.tasks = t64;
+      w.tasks = ctx->d_rtasks64 + cph.rtask_off;
       w.units32 = ctx->d_units32;
-      w.tasks32 = t32;
+      w.tasks32 = ctx->d_rtasks32 + cph.rtask_off;
     }
     if (o.D2 && w.acc_colsC > 0) {  // two accumulator sets must fit the workgroup's LDS
       const size_t nA = ncart_c(w.la), nB = ncart_c(w.lb);
@@ -1741,7 +1775,7 @@ static int run_classes(asuka_jk_ctx* ctx, const EriOut& o, hipStream_t s, bool t
     }
     if (o.counters && cph.nunits > 0 && eri_fast_has_plan(w.la, w.lb, w.lc, w.ld)) {
       hipLaunchKernelGGL(k_count_units, dim3(grid_for(cph.nunits, 4)), dim3(256), 0, ls, *dev,
-                         ctx->d_units + cph.unit_start, cph.nunits, routed ? ctx->d_rf32 + cph.unit_start : nullptr,
+                         ctx->d_units + cph.unit_start, cph.nunits, oo.mixed ? ctx->d_rflag + cph.unit_start : nullptr,
                          ctx->d_col_pair, o.eps_density, o.eps_prim, o.counters + (size_t)kCountStride * i);
       HIP_CHECK(hipGetLastError());
     }
@@ -2136,7 +2170,7 @@ int asuka_jk_autotune(asuka_jk_ctx* ctx, const double* D, int flags, int reps, v
     cp.tuned_ms = std::max(best, 1e-6);
   }
   assign_streams(ctx);
-  return route_task_layout(ctx);  // the cuts may have changed
+  return ctx->d_rflag ? route_task_layout(ctx, s) : ASUKA_OK;  // the cuts may have changed
 }
 
 int asuka_jk_tuning_get(const asuka_jk_ctx* ctx, int32_t* rows, int cap) {
@@ -2176,7 +2210,7 @@ int asuka_jk_tuning_set(asuka_jk_ctx* ctx, const int32_t* rows, int n, void* str
     }
   }
   assign_streams(ctx);
-  return route_task_layout(ctx);  // the cuts may have changed
+  return ctx->d_rflag ? route_task_layout(ctx, s) : ASUKA_OK;  // the cuts may have changed
 }
 
 int asuka_jk_last_timing(asuka_jk_ctx* ctx, double* ms, int64_t* nlaunch) {
