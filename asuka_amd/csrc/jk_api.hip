@@ -471,7 +471,7 @@ __global__ __launch_bounds__(256) void k_count_units(const DevBasis b, const Wav
     long long nev = 0;
     if (active && ur.ni > 0) {
       const int cd0 = b.pp_start[Qp], ncd = min(b.pp_count[Qp], ur.j1);
-      const double kcut = eps_prim / b.ppf[b.pp_start[P] + ur.i0].q;
+      const double kcut = eps_prim / b.ppf[b.pp_start[P]].q;  // the pair's largest, as the kernels
       int j = ur.j0;
       while (j < ncd && !(b.ppf[cd0 + j].q < kcut)) ++j;
       nev = (long long)ur.ni * max(0, j - ur.j0);

@@ -371,7 +371,9 @@ __device__ __forceinline__ void run_chunk(ArgP ap, const Bra& br, int col, const
   // sorted by their Schwarz bound q (largest first). nab (uniform, from the
   // wave unit) already leaves out the bra pairs whose q times the largest
   // ket-pair bound of the unit is below eps_prim; a lane leaves its ket loop
-  // at the first ket pair whose q times the largest bra bound is below it.
+  // at the first ket pair whose q times the largest bra bound is below it (the
+  // shell pair's largest, also in a slice that starts further down: a cut at
+  // the slice's own would drop more, 1e-11 of J and K in sum over a cluster).
   // Every skipped primitive quartet adds less than eps_prim to each integral.
   if (nab > 0) {
     const void* pp = ap->pp;
@@ -379,9 +381,9 @@ __device__ __forceinline__ void run_chunk(ArgP ap, const Bra& br, int col, const
     const float* kpf = ap->kpf;
     CT kcut;
     if constexpr (sizeof(CT) == 8)
-      kcut = ap->eps_prim * rcp_nr(((const ASUKA_CONST PrimPairF*)pp)[ab0].q);
+      kcut = ap->eps_prim * rcp_nr(((const ASUKA_CONST PrimPairF*)pp)[br.ab0].q);
     else
-      kcut = CT(ap->eps_prim * rcp_nr((double)((const ASUKA_CONST PrimPairF32*)pp)[ab0].q));
+      kcut = CT(ap->eps_prim * rcp_nr((double)((const ASUKA_CONST PrimPairF32*)pp)[br.ab0].q));
     // slot rows of the unit's block: the lanes' j-th primitive pairs
     const long long ks0 = cl(ap->kpoff, col >> 6);
     Prim<CT> Yn;
