@@ -372,8 +372,8 @@ __device__ __forceinline__ void run_chunk(ArgP ap, const Bra& br, int col, const
   // wave unit) already leaves out the bra pairs whose q times the largest
   // ket-pair bound of the unit is below eps_prim; a lane leaves its ket loop
   // at the first ket pair whose q times the largest bra bound is below it (the
-  // shell pair's largest, also in a slice that starts further down: a cut at
-  // the slice's own would drop more, 1e-11 of J and K in sum over a cluster).
+  // shell pair's largest, also in a slice that starts further down, so that a
+  // slice leaves out no more than the uncut unit does).
   // Every skipped primitive quartet adds less than eps_prim to each integral.
   if (nab > 0) {
     const void* pp = ap->pp;

@@ -70,8 +70,7 @@ def test_slices_skip_the_same_primitive_quartets(gpu):
     """A 4-water cluster alone (cut into slices) and beside a 12-water one in a
     batch (whose units are longer, so it is cut less) leave out the same
     primitive quartets. The sums then differ by their order alone: about 4e4
-    terms into elements up to 1e2 give under 1e-12 (1.6e-13 measured with no
-    slices at all); a cut at each slice's own largest bound gave 1.4e-10."""
+    terms into elements up to 1e2, under 2e-12 in the positions drawn here."""
     import torch
 
     from asuka_amd.basis import build_ao_basis_cart
