@@ -548,8 +548,8 @@ struct asuka_jk_ctx {
   std::vector<WaveUnit> h_units;  // host copies of the wave units and ket lists
   // routing of mixed builds: per wave unit FP64/FP32 flags (nunits + 1
   // entries, the last 0), their exclusive sums, the two routed unit lists, the
-  // remapped row tasks of every class pair (rtask_cap entries each) and the
-  // scan scratch
+  // row tasks of the routed class pairs (d_rtasks: one of rlayouts), their
+  // remapped copies (rtask_cap entries each) and the scan scratch
   unsigned long long *d_rflag = nullptr, *d_rpos = nullptr;
   // per ket position: Q of the pair (0 for padding) and, per build, the
   // running max of the pairs' max|D| from the position's 64-block start
@@ -558,7 +558,8 @@ struct asuka_jk_ctx {
   int* d_pos_of_sp = nullptr;      // position of each shell pair in the ket lists (-1: none)
   std::vector<int> h_shell_lao;    // host copy of DevBasis::shell_lao
   WaveUnit *d_units64 = nullptr, *d_units32 = nullptr;
-  RowTask *d_rtasks = nullptr, *d_rtasks64 = nullptr, *d_rtasks32 = nullptr;  // all routed class pairs' row tasks
+  RowTask *d_rtasks = nullptr, *d_rtasks64 = nullptr, *d_rtasks32 = nullptr;
+  std::vector<std::pair<std::vector<const RowTask*>, RowTask*>> rlayouts;  // the class pairs' cuts, their list
   long long nrtasks = 0;
   long long rtask_cap = 0;
   void* d_scan_tmp = nullptr;
@@ -641,35 +642,58 @@ static bool row_acc_fits(const asuka_jk_ctx* ctx, int la, int lb, int lc, int ld
   return bytes <= std::min(ctx->row_acc_max, ctx->lds_per_group - root_table_lds(nr) - 1024);
 }
 
-// The routed class pairs' row tasks (of their current cuts) end to end, with
-// the room their remapped copies take, which grows when a cut needs more
-// (context creation and the autotuner's re-cuts; never during a build).
+// The routed class pairs' row tasks (of their current cuts) end to end, and the
+// room their remapped copies take, which grows when a cut needs more (context
+// creation and re-tuning; never during a build). A list that a build may have
+// read is never written again: graphs captured before a re-tuning hold its
+// address and offsets, and a build may still run on another stream. Each
+// combination of cuts therefore gets a list of its own, kept for the life of
+// the context and used again when the cuts return to it, as the cuts are.
 static int route_task_layout(asuka_jk_ctx* ctx, hipStream_t s) {
+  ctx->d_rtasks = nullptr;  // no mixed build splits class pairs until the list is whole
   long long tot = 0;
+  std::vector<const RowTask*> key;
   for (auto& cp : ctx->cps) {
     cp.rtask_off = tot;
-    if (cp.route) tot += cp.ntasks;
+    if (!cp.route) continue;
+    key.push_back(cp.d_tasks_own ? cp.d_tasks_own : ctx->d_tasks + cp.task_start);
+    tot += cp.ntasks;
   }
   ctx->nrtasks = tot;
-  const long long cap = std::max<long long>(1, tot);
-  if (cap > ctx->rtask_cap) {
-    for (RowTask** p : {&ctx->d_rtasks, &ctx->d_rtasks64, &ctx->d_rtasks32}) {
-      RowTask* a = nullptr;
-      HIP_CHECK(hipMalloc(&a, sizeof(RowTask) * (size_t)cap));
-      ctx->owned.push_back(a);
-      *p = a;
+  for (const auto& l : ctx->rlayouts)
+    if (l.first == key) {
+      ctx->d_rtasks = l.second;  // rtask_cap has been at least tot since it was made
+      return ASUKA_OK;
     }
+  const long long cap = std::max<long long>(1, tot);
+  auto alloc = [&](RowTask** p) {
+    const hipError_t e = hipMalloc((void**)p, sizeof(RowTask) * (size_t)cap);
+    if (e == hipSuccess) ctx->owned.push_back(*p);
+    return e;
+  };
+  if (cap > ctx->rtask_cap) {
+    RowTask *a = nullptr, *b = nullptr;
+    HIP_CHECK(alloc(&a));
+    HIP_CHECK(alloc(&b));
+    ctx->d_rtasks64 = a;
+    ctx->d_rtasks32 = b;
     ctx->rtask_cap = cap;
   }
+  RowTask* list = nullptr;
+  HIP_CHECK(alloc(&list));
+  size_t k = 0;
   for (auto& cp : ctx->cps) {
-    if (!cp.route || cp.ntasks <= 0) continue;
-    const RowTask* t = cp.d_tasks_own ? cp.d_tasks_own : ctx->d_tasks + cp.task_start;
+    if (!cp.route) continue;
+    const RowTask* t = key[k++];
+    if (cp.ntasks <= 0) continue;
     const long long g = std::min<long long>((cp.ntasks + 255) / 256, 65535);
     hipLaunchKernelGGL(k_shift_tasks, dim3((unsigned)g), dim3(256), 0, s, t, cp.ntasks, (int)cp.unit_start,
-                       ctx->d_rtasks + cp.rtask_off);
+                       list + cp.rtask_off);
   }
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipStreamSynchronize(s));
+  ctx->rlayouts.emplace_back(std::move(key), list);
+  ctx->d_rtasks = list;
   return ASUKA_OK;
 }
 
@@ -1704,7 +1728,7 @@ static int run_classes(asuka_jk_ctx* ctx, const EriOut& o, hipStream_t s, bool t
   // launches, and the units split (in order) into an FP64 and an FP32 list, so
   // each kernel of a class pair walks only its own units.
   const long long nu_all = (long long)ctx->h_units.size();
-  const bool routed = o.mixed && ctx->d_rflag && nu_all > 0;
+  const bool routed = o.mixed && ctx->d_rtasks && nu_all > 0;
   if (routed) {
     hipLaunchKernelGGL(k_pos_dmax, dim3((unsigned)ctx->nblk), dim3(64), 0, s, ctx->d_col_pair, dev->Dsp,
                        ctx->d_dmaxcol);
@@ -2036,14 +2060,15 @@ int asuka_jk_build_batched(int nmol, asuka_jk_ctx* const* ctxs, const double* co
 static int recut_tasks(asuka_jk_ctx* ctx, int i, int task_units, hipStream_t s) {
   ClassPairHost& cp = ctx->cps[i];
   if (task_units == cp.task_units) return ASUKA_OK;
-  cp.task_units = task_units;
   if (task_units == cp.task_units0) {
+    cp.task_units = task_units;
     cp.d_tasks_own = nullptr;
     cp.ntasks = cp.ntasks0;
     return ASUKA_OK;
   }
   for (const auto& c : cp.cuts)
     if (c.first == task_units) {
+      cp.task_units = task_units;
       cp.d_tasks_own = c.second.first;
       cp.ntasks = c.second.second;
       return ASUKA_OK;
@@ -2055,6 +2080,7 @@ static int recut_tasks(asuka_jk_ctx* ctx, int i, int task_units, hipStream_t s) 
   ctx->owned.push_back(d);
   HIP_CHECK(hipMemcpyAsync(d, tk.data(), sizeof(RowTask) * tk.size(), hipMemcpyHostToDevice, s));
   HIP_CHECK(hipStreamSynchronize(s));
+  cp.task_units = task_units;
   cp.d_tasks_own = d;
   cp.ntasks = (long long)tk.size();
   cp.cuts.push_back({task_units, {d, cp.ntasks}});
@@ -2140,6 +2166,7 @@ int asuka_jk_autotune(asuka_jk_ctx* ctx, const double* D, int flags, int reps, v
     return ASUKA_OK;
   };
   int rc = ASUKA_OK;
+  ctx->d_rtasks = nullptr;  // the cuts change: no list holds until route_task_layout, also after an error
   for (size_t ii = 0; ii < ctx->cps.size(); ++ii) {
     const int i = (int)ii;
     ClassPairHost& cp = ctx->cps[i];
@@ -2199,6 +2226,7 @@ int asuka_jk_tuning_set(asuka_jk_ctx* ctx, const int32_t* rows, int n, void* str
     if (r[4] != 4 && r[4] != 8) return fail(ASUKA_E_INVALID, "wavefronts per workgroup must be 4 or 8");
     if (r[5] < 1 || r[5] > 1024) return fail(ASUKA_E_INVALID, "units per task must be in [1, 1024]");
   }
+  ctx->d_rtasks = nullptr;  // the cuts change: no list holds until route_task_layout, also after an error
   for (int k = 0; k < n; ++k) {
     const int32_t* r = rows + 8 * k;
     for (size_t i = 0; i < ctx->cps.size(); ++i) {

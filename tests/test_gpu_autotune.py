@@ -87,3 +87,46 @@ def test_tuning_errors(gpu):
                          "tuned_ms": 0.0}])
     with pytest.raises(ValueError, match="must be"):
         ctx.autotune(np.zeros((3, 3)))
+
+
+def test_graph_of_mixed_build_survives_retuning(gpu):
+    """A mixed build captured under one table replays unchanged after tables
+    with fewer and with more row tasks (lists that replaced the captured ones in
+    place would hand its kernels other class pairs' units). Replays and eager
+    builds differ by the order of their sums: fewer than 1e5 terms below 10 in
+    elements below 1e2, 1e-12."""
+    from asuka_amd.hf.direct_jk import direct_JK
+
+    torch = gpu
+    ao, ctx = _ctx(water_cluster(3, 5, "cc-pVDZ"), tau_mixed=1e-3)
+    C = np.linalg.qr(np.random.default_rng(7).standard_normal((ao.nao, 15)))[0]
+    D = torch.tensor(2.0 * C @ C.T, device="cuda")
+    default = ctx.tuning()
+
+    def units(n):
+        return [dict(t, units_per_task=n) for t in default]
+
+    ctx.set_tuning(units(1))  # as many tasks as units
+    stats = {}
+    ref = direct_JK(ctx, D, mixed_precision=True, stats=stats)
+    assert 0 < sum(c["quartets_fp32"] for c in stats["class_counts"]) < stats["direct_jk_evaluated"]
+    out = tuple(torch.empty_like(x) for x in ref)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        direct_JK(ctx, D, mixed_precision=True, out=out)
+    torch.cuda.current_stream().wait_stream(s)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        direct_JK(ctx, D, mixed_precision=True, out=out)
+    for table in (default, units(4), units(1), default):
+        ctx.set_tuning(table)
+        eager = direct_JK(ctx, D, mixed_precision=True)
+        for x in out:
+            x.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        for x, y, r in zip(out, eager, ref):
+            assert float((x - r).abs().max()) < 1e-12 and float((y - r).abs().max()) < 1e-12
