@@ -134,38 +134,88 @@ static inline long long slice_min(int nroots) { return std::max(2, 48 / (nroots 
 // (H2O)5 two densities 2033 / 1983 / 1816 / 1783 / 1782, (H2O)14 11200 / 11180
 // / 11241 / 11479 / 12289, (H2O)8 cc-pVTZ 48.3 / 48.2 / 48.3 / 50.9 / 53.0 ms.
 // The largest class pair is split from kRouteMinLargest on, so that a mixed
-// build does run FP32 kernels from two molecules on (+40 us at (H2O)3).
+// build does run FP32 kernels from two molecules on (+40 us at (H2O)3). In a
+// batch the items of each molecule decide for its own units, counted as a
+// context of its own would have them, and units that may go to FP32 are sliced
+// as there: beside others a molecule's mixed J and K are those of a context of
+// its own but for the order of the FP64 sums.
 static constexpr long long kRouteMin = 16384;
 static constexpr long long kRouteMinLargest = 2048;
 
-// blk_k: largest primitive-pair count of each 64-position ket block.
-static void slice_units(const std::vector<int>& blk_k, ClassPairHost& cp, std::vector<WaveUnit>& units) {
+// Slices of a unit, bra blocks x ket blocks, for at most `most` primitive
+// quartets each (kcd: the longest primitive-pair list of its kets).
+static std::pair<int, int> slices_of(const WaveUnit& u, int kcd, long long most) {
+  const int ni = (int)u.i1;
+  const long long w = (long long)ni * kcd;
+  if (w <= most || ni >= kUnitAll || kcd >= kUnitAll) return {1, 1};
+  const long long n = (w + most - 1) / most;
+  const int si = (int)std::min<long long>(ni, n);
+  return {si, (int)std::min<long long>(kcd, (n + si - 1) / si)};
+}
+
+// The longest slice a class pair's units are cut into, from the work of all of
+// them (primitive quartets times wave items).
+static long long slice_most(const ClassPairHost& cp, long long total) {
+  return std::max(slice_min((cp.la + cp.lb + cp.lc + cp.ld) / 2 + 1), total / kSliceWaves);
+}
+
+// Per molecule, of a class pair's unsliced units: their work (primitive
+// quartets times wave items), the longest one's primitive quartets and the wave
+// items they are cut into in a context of the molecule's own. blk_k: largest
+// primitive-pair count of each 64-position ket block; mol: the molecule of a
+// shell pair.
+struct MolWork {
+  std::vector<long long> total, longest, items;
+};
+template <typename F>
+static MolWork mol_work(const std::vector<int>& blk_k, const ClassPairHost& cp, const std::vector<WaveUnit>& units,
+                        int nmol, F&& mol) {
+  const std::vector<long long> zero((size_t)nmol, 0);
+  MolWork r{zero, zero, zero};
   const int nit = eri_fast_nch(cp.la, cp.lb, cp.lc, cp.ld);
-  if (nit <= 0 || cp.rows.empty()) return;
-  const size_t u0 = (size_t)cp.unit_start;
-  auto work = [&](const WaveUnit& u) { return (long long)u.i1 * blk_k[(size_t)u.col >> 6]; };  // primitive quartets
-  long long total = 0, longest = 0;
-  for (size_t k = u0; k < units.size(); ++k) {
-    const long long w = work(units[k]);
-    total += w * nit;
-    longest = std::max(longest, w);
+  if (nit <= 0) return r;
+  const size_t u0 = (size_t)cp.unit_start, u1 = u0 + (size_t)cp.nunits;
+  for (size_t k = u0; k < u1; ++k) {
+    const int m = mol(units[k].P);
+    const long long w = (long long)units[k].i1 * blk_k[(size_t)units[k].col >> 6];
+    r.total[m] += w * nit;
+    r.longest[m] = std::max(r.longest[m], w);
+    r.items[m] += nit;
   }
-  const long long most = std::max(slice_min((cp.la + cp.lb + cp.lc + cp.ld) / 2 + 1), total / kSliceWaves);
-  if (longest <= most) return;
-  std::vector<WaveUnit> out;
+  bool cut = false;
+  for (int m = 0; m < nmol; ++m) cut = cut || r.longest[m] > slice_most(cp, r.total[m]);
+  if (!cut) return r;
+  r.items = zero;
+  for (size_t k = u0; k < u1; ++k) {
+    const int m = mol(units[k].P);
+    const auto sl = slices_of(units[k], blk_k[(size_t)units[k].col >> 6], slice_most(cp, r.total[m]));
+    r.items[m] += (long long)sl.first * sl.second * nit;
+  }
+  return r;
+}
+
+// Appends a class pair's units to out, with cut in slices of at most most(P)
+// primitive quartets for bra pair P; the class pair's rows, unit_start and
+// nunits then name the slices.
+template <typename F>
+static void slice_units(const std::vector<int>& blk_k, ClassPairHost& cp, const std::vector<WaveUnit>& units, bool cut,
+                        F&& most, std::vector<WaveUnit>& out) {
+  const size_t u0 = (size_t)cp.unit_start, o0 = out.size();
+  cp.unit_start = (long long)o0;
+  if (!cut) {
+    out.insert(out.end(), units.begin() + u0, units.begin() + u0 + (size_t)cp.nunits);
+    return;
+  }
   for (auto& row : cp.rows) {
-    const int first = (int)out.size();
+    const int first = (int)(out.size() - o0);
     for (int k = row.first; k < row.first + row.second; ++k) {
       const WaveUnit u = units[u0 + k];
-      const int ni = (int)u.i1;
-      const long long w = work(u);
-      const int kcd = blk_k[(size_t)u.col >> 6];
-      if (w <= most || ni >= kUnitAll || kcd >= kUnitAll) {
+      const int ni = (int)u.i1, kcd = blk_k[(size_t)u.col >> 6];
+      const auto [si, sj] = slices_of(u, kcd, most(u.P));
+      if (si * sj == 1) {
         out.push_back(u);
         continue;
       }
-      const long long n = (w + most - 1) / most;
-      const int si = (int)std::min<long long>(ni, n), sj = (int)std::min<long long>(kcd, (n + si - 1) / si);
       for (int a = 0; a < si; ++a)
         for (int c = 0; c < sj; ++c) {
           WaveUnit v = u;
@@ -177,10 +227,9 @@ static void slice_units(const std::vector<int>& blk_k, ClassPairHost& cp, std::v
           out.push_back(v);
         }
     }
-    row = {first, (int)out.size() - first};
+    row = {first, (int)(out.size() - o0) - first};
   }
-  units.resize(u0);
-  units.insert(units.end(), out.begin(), out.end());
+  cp.nunits = (long long)(out.size() - o0);
 }
 
 // Row tasks of a class pair: each row's wave units cut into
@@ -397,16 +446,17 @@ __global__ void k_pos_dmax(const int* __restrict__ col, const double* __restrict
 // unit is then below tau: the FP32 kernel's share), 1 otherwise, 0 when it is
 // below eps_density (every quartet density-screened): one sum counts both. A
 // unit kept by the bound whose quartets are all screened is skipped in the
-// kernel, which tests each quartet itself.
+// kernel, which tests each quartet itself. allow (null: every unit): units of
+// a batch whose molecule has enough of them for FP32 (kRouteMin).
 __global__ void k_route_units(DevBasis b, const WaveUnit* __restrict__ units, const double* __restrict__ qcol,
-                              const double* __restrict__ dmaxcol, long long nunits, double eps_density, double tau,
-                              unsigned long long* flags) {
+                              const double* __restrict__ dmaxcol, const unsigned char* __restrict__ allow,
+                              long long nunits, double eps_density, double tau, unsigned long long* flags) {
   for (long long u = blockIdx.x * (long long)blockDim.x + threadIdx.x; u < nunits;
        u += (long long)gridDim.x * blockDim.x) {
     const WaveUnit un = units[u];
     const double hi = (b.Q[un.P] * qcol[un.col]) * fmax(b.Dsp[un.P], dmaxcol[un.col + un.ncol - 1]);
     const bool any = un.ncol > 0 && (eps_density > 0.0 ? hi >= eps_density : true);
-    flags[u] = !any ? 0ull : hi < tau ? 1ull << 32 : 1ull;
+    flags[u] = !any ? 0ull : hi < tau && (!allow || allow[u]) ? 1ull << 32 : 1ull;
   }
 }
 
@@ -551,6 +601,7 @@ struct asuka_jk_ctx {
   // row tasks of the routed class pairs (d_rtasks: one of rlayouts), their
   // remapped copies (rtask_cap entries each) and the scan scratch
   unsigned long long *d_rflag = nullptr, *d_rpos = nullptr;
+  unsigned char* d_rallow = nullptr;  // batch contexts: k_route_units' allow
   // per ket position: Q of the pair (0 for padding) and, per build, the
   // running max of the pairs' max|D| from the position's 64-block start
   double *d_qcol = nullptr, *d_dmaxcol = nullptr;
@@ -1306,8 +1357,7 @@ static int ctx_build(const asuka_basis_desc* bd, const std::vector<int>* shell_m
   std::vector<int> col_all, row_pair_all;
   std::vector<long long> row_off_all;
   std::vector<Segment> segs;
-  std::vector<WaveUnit> units;
-  std::vector<RowTask> tasks;
+  std::vector<WaveUnit> whole;  // wave units before slicing
   for (size_t c = 0; c < cls_pairs.size(); ++c) {
     std::vector<int> kvals;
     for (int sp : cls_pairs[c]) kvals.push_back(kbucket(ctx->pp_count[sp]));
@@ -1347,10 +1397,8 @@ static int ctx_build(const asuka_basis_desc* bd, const std::vector<int>* shell_m
       cp.lc = cls_la[Y];
       cp.ld = cls_lb[Y];
       cp.seg_start = (int)segs.size();
-      cp.unit_start = (long long)units.size();
-      cp.task_start = (long long)tasks.size();
+      cp.unit_start = (long long)whole.size();
       const int nroots = (cp.la + cp.lb + cp.lc + cp.ld) / 2 + 1;
-      int task_units = kTaskUnits;
       {  // LDS row accumulators and workgroup size of this class pair
         const int cC = ctx->nlao[cp.lc], cD = (cp.lc == cp.ld) ? 0 : ctx->nlao[cp.ld];
         const size_t bytes = sizeof(double) * (size_t)(ncart_c(cp.la) * ncart_c(cp.lb) +
@@ -1359,7 +1407,7 @@ static int ctx_build(const asuka_basis_desc* bd, const std::vector<int>* shell_m
         cp.acc_colsC = fits ? cC : 0;
         cp.acc_colsD = fits ? cD : 0;
         cp.wpg = (fits && bytes > kRowAccSmallBytes) ? 8 : 4;
-        cp.task_units = task_units;
+        cp.task_units = cp.task_units0 = kTaskUnits;
       }
       long long padded = 0;
       for (int m = 0; m < nmol; ++m)
@@ -1402,7 +1450,7 @@ static int ctx_build(const asuka_basis_desc* bd, const std::vector<int>* shell_m
             {
               // the row's wave units (cut into row tasks below)
               const int nu = (int)((len + 63) / 64);
-              cp.rows.emplace_back((int)(units.size() - cp.unit_start), nu);
+              cp.rows.emplace_back((int)(whole.size() - cp.unit_start), nu);
               for (long long c0 = 0; c0 < len; c0 += 64) {
                 const int nc = (int)std::min<long long>(64, len - c0);
                 int nabu = ctx->pp_count[P];
@@ -1424,7 +1472,7 @@ static int ctx_build(const asuka_basis_desc* bd, const std::vector<int>* shell_m
                 wu.tail = 1;
                 wu.i1 = (unsigned)std::min(nabu, kUnitAll);
                 wu.j1 = kUnitAll;
-                units.push_back(wu);
+                whole.push_back(wu);
               }
             }
           }
@@ -1452,15 +1500,7 @@ static int ctx_build(const asuka_basis_desc* bd, const std::vector<int>* shell_m
         }
       }
       cp.nseg = (int)segs.size() - cp.seg_start;
-      slice_units(blk_k, cp, units);
-      cp.nunits = (long long)units.size() - cp.unit_start;
-      {
-        const std::vector<RowTask> tk = make_tasks(cp, units.data() + cp.unit_start, col_all, ctx->pp_count, task_units);
-        tasks.insert(tasks.end(), tk.begin(), tk.end());
-        cp.ntasks = cp.ntasks0 = (long long)tk.size();
-        cp.task_units0 = task_units;
-      }
-
+      cp.nunits = (long long)whole.size() - cp.unit_start;
       if (cp.nseg == 0) continue;
       cp.nwork = padded;
       cp.nprim_roots = cp.nprim_quartets * nroots;
@@ -1475,20 +1515,57 @@ static int ctx_build(const asuka_basis_desc* bd, const std::vector<int>* shell_m
       ctx->ntasks += cp.nquartets;
     }
   }
-  {  // class pairs that mixed builds split (kRouteMin)
-    auto items = [](const ClassPairHost& c) { return c.nunits * eri_fast_nch(c.la, c.lb, c.lc, c.ld); };
-    ClassPairHost* big = nullptr;
-    for (auto& cp : ctx->cps) {
-      cp.route = items(cp) > (opts->tau_mixed > 0.0 ? 0 : kRouteMin);
-      if (!big || items(cp) > items(*big)) big = &cp;
+  // Class pairs that mixed builds split (kRouteMin), by molecule; the slices of
+  // the units (of a molecule that splits the class pair as in a context of its
+  // own: an FP32 unit's sum depends on its slices); the row tasks.
+  std::vector<WaveUnit> units;
+  std::vector<RowTask> tasks;
+  std::vector<unsigned char> allow;  // batch contexts, per unit: its molecule splits the class pair
+  {
+    const size_t n = ctx->cps.size();
+    auto mol_of = [&](int sp) { return nmol > 1 ? ctx->shell_mol[ctx->sp_A[sp]] : 0; };
+    std::vector<MolWork> work;
+    for (const auto& cp : ctx->cps) work.push_back(mol_work(blk_k, cp, whole, nmol, mol_of));
+    std::vector<std::vector<unsigned char>> split(n, std::vector<unsigned char>((size_t)nmol, 0));
+    for (int m = 0; m < nmol; ++m) {
+      size_t big = 0;
+      for (size_t c = 0; c < n; ++c) {
+        split[c][m] = work[c].items[m] > (opts->tau_mixed > 0.0 ? 0 : kRouteMin);
+        if (work[c].items[m] > work[big].items[m]) big = c;
+      }
+      if (n > 0 && work[big].items[m] > kRouteMinLargest) split[big][m] = 1;
     }
-    if (big && items(*big) > kRouteMinLargest) big->route = true;
+    std::vector<std::vector<long long>> most(n, std::vector<long long>((size_t)nmol));  // longest slice
+    std::vector<unsigned char> cut(n, 0);
+    for (size_t c = 0; c < n; ++c) {
+      const ClassPairHost& cp = ctx->cps[c];
+      const long long all = slice_most(cp, std::accumulate(work[c].total.begin(), work[c].total.end(), 0ll));
+      for (int m = 0; m < nmol; ++m) {
+        most[c][m] = split[c][m] ? slice_most(cp, work[c].total[m]) : all;
+        if (work[c].longest[m] > most[c][m]) cut[c] = 1;
+      }
+    }
+    const bool keep = std::none_of(cut.begin(), cut.end(), [](unsigned char x) { return x != 0; });
+    if (keep) units = std::move(whole);  // large contexts: nothing to cut
+    for (size_t c = 0; c < n; ++c) {
+      ClassPairHost& cp = ctx->cps[c];
+      if (!keep) slice_units(blk_k, cp, whole, cut[c], [&](int P) { return most[c][mol_of(P)]; }, units);
+      for (unsigned char x : split[c]) cp.route = cp.route || x;
+      const std::vector<RowTask> tk = make_tasks(cp, units.data() + cp.unit_start, col_all, ctx->pp_count, cp.task_units);
+      cp.task_start = (long long)tasks.size();
+      tasks.insert(tasks.end(), tk.begin(), tk.end());
+      cp.ntasks = cp.ntasks0 = (long long)tk.size();
+      if (nmol > 1)
+        for (long long u = 0; u < cp.nunits; ++u)
+          allow.push_back(split[c][mol_of(units[(size_t)(cp.unit_start + u)].P)]);
+    }
   }
   assign_streams(ctx);
   col_all.resize((col_all.size() + 63) / 64 * 64, -1);
   if ((rc = pos_layout(ctx, col_all))) return rc;
   if ((rc = dev_upload(&ctx->d_segs, segs, own, s))) return rc;
   if ((rc = dev_upload(&ctx->d_units, units, own, s))) return rc;
+  if (!allow.empty() && (rc = dev_upload(&ctx->d_rallow, allow, own, s))) return rc;
   if ((rc = dev_upload(&ctx->d_tasks, tasks, own, s))) return rc;
   if ((rc = dev_upload(&ctx->d_row_pair, row_pair_all, own, s))) return rc;
   if ((rc = dev_upload(&ctx->d_row_off, row_off_all, own, s))) return rc;
@@ -1734,7 +1811,7 @@ static int run_classes(asuka_jk_ctx* ctx, const EriOut& o, hipStream_t s, bool t
                        ctx->d_dmaxcol);
     HIP_CHECK(hipGetLastError());
     hipLaunchKernelGGL(k_route_units, dim3(grid_for(nu_all, 256)), dim3(256), 0, s, *dev, ctx->d_units, ctx->d_qcol,
-                       ctx->d_dmaxcol, nu_all, o.eps_density, o.tau_mixed, ctx->d_rflag);
+                       ctx->d_dmaxcol, ctx->d_rallow, nu_all, o.eps_density, o.tau_mixed, ctx->d_rflag);
     HIP_CHECK(hipGetLastError());
     size_t tb = ctx->scan_tmp_bytes;
     HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(ctx->d_scan_tmp, tb, ctx->d_rflag, ctx->d_rpos, (int)(nu_all + 1), s));

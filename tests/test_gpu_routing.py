@@ -35,3 +35,30 @@ def test_split_class_pairs(gpu, n, basis, tau, split):
     h = np.eye(ao.nao)
     F, F0 = (direct_fock_rhf(ctx, D, h, mixed_precision=m) for m in (True, False))
     assert float((F - F0).abs().max()) < 2 * tol
+
+
+def test_split_does_not_depend_on_the_batch(gpu):
+    """Default mixed builds of a batch equal those of one-molecule contexts to
+    the order of the FP64 sums (fewer than 1e5 terms below 10 in elements below
+    1e2: 1e-12), with molecules that split none, some and most of their class
+    pairs; with the class pairs' sizes taken over the batch, or FP32 units
+    sliced by its work, they differ by 1e-11 to 1e-10."""
+    import torch
+
+    from asuka_amd.hf.direct_jk import direct_JK, direct_JK_batched, make_direct_jk_batch_context, \
+        make_direct_jk_context
+
+    aos, Ds = [], []
+    for n, seed in ((1, 8), (4, 3), (12, 17), (3, 2)):
+        ao, _ = build_ao_basis_cart(water_cluster(n, 1000 + seed, "cc-pVDZ"))
+        C, _ = np.linalg.qr(np.random.default_rng(2000 + seed).standard_normal((ao.nao, 5 * n)))
+        aos.append(ao)
+        Ds.append(torch.tensor(2.0 * C @ C.T, device="cuda"))
+    batch = direct_JK_batched(make_direct_jk_batch_context(aos), Ds, mixed_precision=True)
+    q32 = []
+    for ao, D, got in zip(aos, Ds, batch):
+        st = {}
+        ref = direct_JK(make_direct_jk_context(ao), D, mixed_precision=True, stats=st)
+        q32.append(sum(c["quartets_fp32"] for c in st["class_counts"]))
+        assert all(float((x - y).abs().max()) < 1e-12 for x, y in zip(got, ref)), ao.nao
+    assert q32[0] == 0 < q32[1] < q32[2]
