@@ -118,7 +118,8 @@ struct ClassPairHost {
 // quartets, fewer for more roots (a primitive quartet of a class with n roots
 // costs about n^2 times as much; 24, 96 and 192 / n^2 were measured 9 % faster,
 // 32 % and 65 % slower than 48 for one water, and 2 %, 3 % and 4 % slower for
-// (H2O)7). Large contexts have no such unit and are left alone. Measured with
+// (H2O)7). Large contexts have no such unit and are left alone. Deterministic
+// builds run every unit whole (eri_fast_kernel). Measured with
 // kFillTasks: one water cc-pVDZ, mixed Fock build 2.37 -> 0.60 ms, (H2O)7 FP64
 // 4.66 -> 3.46 ms, (H2O)2 cc-pVTZ J/K 8.7 -> 3.8 ms, (H2O)5 two densities 3.68
 // -> 2.41 ms.

@@ -830,6 +830,10 @@ __global__ __launch_bounds__(kGroupThreads) void eri_fast_kernel(FastArgs args) 
           WaveUnit u;
         } un;
         un.v = cl((const u32x4*)ap->units, u0 + ui);
+        // a quartet of a deterministic build is rounded once, as a whole: the
+        // last slice of a sliced unit runs all of it, the others nothing
+        if constexpr (FX)
+          if (!un.u.tail || (int)un.u.j1 != kUnitAll) continue;
         const int col = un.u.col;
         // the lane's ket position is col + lane: units start at 64-position
         // block boundaries, so tail lanes read padding positions of the block
@@ -845,7 +849,8 @@ __global__ __launch_bounds__(kGroupThreads) void eri_fast_kernel(FastArgs args) 
         worked = true;
         // inactive lanes (tail, screened) run with an empty primitive loop and no
         // atomics so the wave stays converged for the cross-lane reductions
-        const UnitRange ur = unit_range(un.u, cl(ap->pp_count, br.P), false);
+        UnitRange ur = unit_range(un.u, cl(ap->pp_count, br.P), false);
+        if constexpr (FX) ur = UnitRange{0, ur.i0 + ur.ni, 0, ur.j1};
         dispatch_citem<PL, 0, CT, FX>(chunk, ap, br, col, ur, active, tab, acc);
       }
       if (acc.on) {

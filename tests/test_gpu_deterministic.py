@@ -110,6 +110,25 @@ def test_deterministic_fock_and_multi(gpu):
         assert float((got - want).abs().max()) < 1e-10
 
 
+@pytest.mark.parametrize("nprim", [1, 3, 8, 17])
+def test_deterministic_rounds_a_quartet_once(gpu, nprim):
+    """One s shell: J and K are one contribution each, so a deterministic build
+    is within half a unit of 2^-44 of the ordinary one (and its few ulp of
+    values below 4), however the ordinary build cuts the primitive loops."""
+    from asuka_amd.basis import pack_cart_basis, parse_basis_dict
+    from asuka_amd.hf.direct_jk import direct_JK, make_direct_jk_context
+
+    spec = {"O": [[0] + [[0.25 * 1.9 ** k, 0.2 + 0.6 / (1 + k)] for k in range(nprim)]]}
+    ao = pack_cart_basis([("O", np.array([0.1, -0.2, 0.05]))], parse_basis_dict(spec, ["O"]))
+    ctx = make_direct_jk_context(ao, eps_schwarz=0.0, eps_density=0.0)
+    v = float(direct_JK(ctx, np.ones((1, 1)), mixed_precision=False)[0])
+    for d in np.random.default_rng(nprim).uniform(0.5, 2.0, size=40) / v:
+        ref = direct_JK(ctx, np.array([[d]]), mixed_precision=False)
+        got = direct_JK(ctx, np.array([[d]]), mixed_precision=False, deterministic=True)
+        for x, y in zip(got, ref):
+            assert abs(float(x - y)) <= 2.0 ** -45 + 4e-15
+
+
 def test_batch_builds_reject_deterministic(gpu):
     import ctypes
 
