@@ -100,9 +100,9 @@ struct ClassPairHost {
   int task_units;       // wave units per row task (at most)
   std::vector<std::pair<int, int>> rows;  // (first unit relative to unit_start, units) per bra row
   RowTask* d_tasks_own = nullptr;         // row tasks re-cut by the autotuner (owned by the context)
-  int task_units0 = 0;                    // the cut stored in the context's d_tasks
+  int cut = 0, cut0 = 0;                  // cut_units of the current cut and of the one in the context's d_tasks
   long long ntasks0 = 0;
-  std::vector<std::pair<int, std::pair<RowTask*, long long>>> cuts;  // other cuts made so far
+  std::vector<std::pair<int, std::pair<RowTask*, long long>>> cuts;  // other cuts made so far, by cut_units
   double tuned_ms = 0.0;                  // time of the class pair's launch when tuned (0: not tuned)
   bool route = false;                     // mixed builds route its units to an FP64 and an FP32 launch
   long long rtask_off = 0;                // first of its remapped row tasks (routed mixed builds)
@@ -241,12 +241,15 @@ static void slice_units(const std::vector<int>& blk_k, ClassPairHost& cp, const 
 // one wave item per wavefront, so that its units spread over the chip (1024
 // measured 1-4 % slower below 10 molecules: each task flushes its LDS sums).
 static constexpr long long kFillTasks = 512;
+static int cut_units(const ClassPairHost& cp, int task_units) {
+  const int nit = std::max(1, eri_fast_nch(cp.la, cp.lb, cp.lc, cp.ld));
+  return (int)std::min<long long>(
+      task_units, std::max<long long>((cp.wpg + nit - 1) / nit, (cp.nunits + kFillTasks - 1) / kFillTasks));
+}
 static std::vector<RowTask> make_tasks(const ClassPairHost& cp, const WaveUnit* units, const std::vector<int>& col,
                                        const std::vector<int>& pp_count, int task_units) {
   std::vector<RowTask> tasks;
-  const int nit = std::max(1, eri_fast_nch(cp.la, cp.lb, cp.lc, cp.ld));
-  task_units = (int)std::min<long long>(
-      task_units, std::max<long long>((cp.wpg + nit - 1) / nit, (cp.nunits + kFillTasks - 1) / kFillTasks));
+  task_units = cut_units(cp, task_units);
   for (const auto& r : cp.rows) {
     const int nu = r.second;
     const int ntk = (nu + task_units - 1) / task_units;
@@ -1408,7 +1411,7 @@ static int ctx_build(const asuka_basis_desc* bd, const std::vector<int>* shell_m
         cp.acc_colsC = fits ? cC : 0;
         cp.acc_colsD = fits ? cD : 0;
         cp.wpg = (fits && bytes > kRowAccSmallBytes) ? 8 : 4;
-        cp.task_units = cp.task_units0 = kTaskUnits;
+        cp.task_units = kTaskUnits;
       }
       long long padded = 0;
       for (int m = 0; m < nmol; ++m)
@@ -1556,6 +1559,7 @@ static int ctx_build(const asuka_basis_desc* bd, const std::vector<int>* shell_m
       cp.task_start = (long long)tasks.size();
       tasks.insert(tasks.end(), tk.begin(), tk.end());
       cp.ntasks = cp.ntasks0 = (long long)tk.size();
+      cp.cut = cp.cut0 = cut_units(cp, cp.task_units);
       if (nmol > 1)
         for (long long u = 0; u < cp.nunits; ++u)
           allow.push_back(split[c][mol_of(units[(size_t)(cp.unit_start + u)].P)]);
@@ -1785,6 +1789,24 @@ static hipStream_t stream_of(const asuka_jk_ctx* ctx, const ClassPairHost& cp, h
   return (cp.stream > 0 && cp.stream <= (int)ctx->side.size()) ? ctx->side[cp.stream - 1] : s;
 }
 
+// The precision of every wave unit (o.eps_density, o.tau_mixed, dev.Dsp), and
+// the units split, in order, into an FP64 and an FP32 list, so that each kernel
+// of a split class pair walks only its own.
+static int route_units(asuka_jk_ctx* ctx, const DevBasis& dev, const EriOut& o, hipStream_t s) {
+  const long long n = (long long)ctx->h_units.size();
+  hipLaunchKernelGGL(k_pos_dmax, dim3((unsigned)ctx->nblk), dim3(64), 0, s, ctx->d_col_pair, dev.Dsp, ctx->d_dmaxcol);
+  HIP_CHECK(hipGetLastError());
+  hipLaunchKernelGGL(k_route_units, dim3(grid_for(n, 256)), dim3(256), 0, s, dev, ctx->d_units, ctx->d_qcol,
+                     ctx->d_dmaxcol, ctx->d_rallow, n, o.eps_density, o.tau_mixed, ctx->d_rflag);
+  HIP_CHECK(hipGetLastError());
+  size_t tb = ctx->scan_tmp_bytes;
+  HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(ctx->d_scan_tmp, tb, ctx->d_rflag, ctx->d_rpos, (int)(n + 1), s));
+  hipLaunchKernelGGL(k_scatter_units, dim3(grid_for(n, 256)), dim3(256), 0, s, ctx->d_units, n, ctx->d_rflag,
+                     ctx->d_rpos, ctx->d_units64, ctx->d_units32);
+  HIP_CHECK(hipGetLastError());
+  return ASUKA_OK;
+}
+
 // queue: the class pairs' work-queue heads (the context's, or the static
 // scratch of asuka_jk_build_noalloc); dev: the device tables the kernels read
 static int run_classes(asuka_jk_ctx* ctx, const EriOut& o, hipStream_t s, bool timed, unsigned int* queue = nullptr,
@@ -1802,22 +1824,11 @@ static int run_classes(asuka_jk_ctx* ctx, const EriOut& o, hipStream_t s, bool t
     hipLaunchKernelGGL(k_zero_u32, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, s, queue, nq);
     HIP_CHECK(hipGetLastError());
   }
-  // Mixed builds: the precision vote of every wave unit once, before the
-  // launches, and the units split (in order) into an FP64 and an FP32 list, so
-  // each kernel of a class pair walks only its own units.
-  const long long nu_all = (long long)ctx->h_units.size();
-  const bool routed = o.mixed && ctx->d_rtasks && nu_all > 0;
+  // Mixed builds: the units and row tasks of the split class pairs
+  const bool routed = o.mixed && ctx->d_rtasks && !ctx->h_units.empty();
   if (routed) {
-    hipLaunchKernelGGL(k_pos_dmax, dim3((unsigned)ctx->nblk), dim3(64), 0, s, ctx->d_col_pair, dev->Dsp,
-                       ctx->d_dmaxcol);
-    HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_route_units, dim3(grid_for(nu_all, 256)), dim3(256), 0, s, *dev, ctx->d_units, ctx->d_qcol,
-                       ctx->d_dmaxcol, ctx->d_rallow, nu_all, o.eps_density, o.tau_mixed, ctx->d_rflag);
-    HIP_CHECK(hipGetLastError());
-    size_t tb = ctx->scan_tmp_bytes;
-    HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(ctx->d_scan_tmp, tb, ctx->d_rflag, ctx->d_rpos, (int)(nu_all + 1), s));
-    hipLaunchKernelGGL(k_scatter_units, dim3(grid_for(nu_all, 256)), dim3(256), 0, s, ctx->d_units, nu_all,
-                       ctx->d_rflag, ctx->d_rpos, ctx->d_units64, ctx->d_units32);
+    const int rc = route_units(ctx, *dev, o, s);
+    if (rc) return rc;
     hipLaunchKernelGGL(k_route_tasks, dim3(grid_for(ctx->nrtasks, 256)), dim3(256), 0, s, ctx->d_rtasks, ctx->nrtasks,
                        ctx->d_rpos, ctx->d_rtasks64, ctx->d_rtasks32);
     HIP_CHECK(hipGetLastError());
@@ -1863,7 +1874,6 @@ static int run_classes(asuka_jk_ctx* ctx, const EriOut& o, hipStream_t s, bool t
     w.queue32 = queue + ncp + i;
     oo.mixed = routed && cph.route ? 1 : 0;  // the other class pairs run in FP64
     if (oo.mixed) {
-      w.routed = 1;
       w.units = ctx->d_units64;
       w.tasks = ctx->d_rtasks64 + cph.rtask_off;
       w.units32 = ctx->d_units32;
@@ -2133,24 +2143,24 @@ int asuka_jk_build_batched(int nmol, asuka_jk_ctx* const* ctxs, const double* co
 
 }  // extern "C"
 
-// Row tasks of class pair i re-cut to task_units units (device copy owned by
-// the context; the original cut stays in d_tasks).
+// Row tasks of class pair i re-cut to task_units units for its wavefronts per
+// workgroup (device copy owned by the context; the original cut stays in
+// d_tasks). A cut is known by its cut_units: requests that come to the same
+// are the same cut.
 static int recut_tasks(asuka_jk_ctx* ctx, int i, int task_units, hipStream_t s) {
   ClassPairHost& cp = ctx->cps[i];
-  if (task_units == cp.task_units) return ASUKA_OK;
-  if (task_units == cp.task_units0) {
+  const int cut = cut_units(cp, task_units);
+  auto use = [&](RowTask* d, long long n) {
     cp.task_units = task_units;
-    cp.d_tasks_own = nullptr;
-    cp.ntasks = cp.ntasks0;
+    cp.cut = cut;
+    cp.d_tasks_own = d;
+    cp.ntasks = n;
     return ASUKA_OK;
-  }
+  };
+  if (cut == cp.cut) return use(cp.d_tasks_own, cp.ntasks);
+  if (cut == cp.cut0) return use(nullptr, cp.ntasks0);
   for (const auto& c : cp.cuts)
-    if (c.first == task_units) {
-      cp.task_units = task_units;
-      cp.d_tasks_own = c.second.first;
-      cp.ntasks = c.second.second;
-      return ASUKA_OK;
-    }
+    if (c.first == cut) return use(c.second.first, c.second.second);
   const std::vector<RowTask> tk =
       make_tasks(cp, ctx->h_units.data() + cp.unit_start, ctx->h_col, ctx->pp_count, task_units);
   RowTask* d = nullptr;
@@ -2158,11 +2168,8 @@ static int recut_tasks(asuka_jk_ctx* ctx, int i, int task_units, hipStream_t s) 
   ctx->owned.push_back(d);
   HIP_CHECK(hipMemcpyAsync(d, tk.data(), sizeof(RowTask) * tk.size(), hipMemcpyHostToDevice, s));
   HIP_CHECK(hipStreamSynchronize(s));
-  cp.task_units = task_units;
-  cp.d_tasks_own = d;
-  cp.ntasks = (long long)tk.size();
-  cp.cuts.push_back({task_units, {d, cp.ntasks}});
-  return ASUKA_OK;
+  cp.cuts.push_back({cut, {d, (long long)tk.size()}});
+  return use(d, (long long)tk.size());
 }
 
 // Applies (wavefronts per workgroup, units per task, LDS accumulators) to class pair i.
@@ -2210,8 +2217,23 @@ int asuka_jk_autotune(asuka_jk_ctx* ctx, const double* D, int flags, int reps, v
   o.K = tjk + nn;
   o.eps_density = ctx->eps_density;
   o.eps_prim = ctx->eps_schwarz > 0.0 ? ctx->eps_prim : 0.0;
-  o.mixed = (flags & ASUKA_JK_MIXED) ? 1 : 0;
   o.tau_mixed = ctx->tau_mixed;
+  // mixed: the units routed for D as in a build, and room for a class pair's
+  // row tasks (at most one a unit) in the whole list and in the two routed ones
+  const bool mixed = (flags & ASUKA_JK_MIXED) && ctx->d_rflag;
+  long long tmax = 1;
+  RowTask* rt = nullptr;
+  struct FreeT {
+    RowTask** p;
+    ~FreeT() { (void)hipFree(*p); }
+  } free_rt{&rt};
+  if (mixed) {
+    const int rc = route_units(ctx, ctx->dev, o, s);
+    if (rc) return rc;
+    for (const auto& cp : ctx->cps)
+      if (cp.route) tmax = std::max(tmax, cp.nunits);
+    HIP_CHECK(hipMalloc(&rt, sizeof(RowTask) * 3 * (size_t)tmax));
+  }
   if (ctx->nblk > 0) {  // the ket-position and flush buffers, as in a build (their contents are discarded)
     o.jblk = ctx->d_jblk;
     o.Jpos = ctx->d_jpos;
@@ -2224,8 +2246,21 @@ int asuka_jk_autotune(asuka_jk_ctx* ctx, const double* D, int flags, int reps, v
   // median of reps timed launches (after one untimed) of class pair i as it is now set up
   auto time_class = [&](int i, double* ms) -> int {
     std::vector<float> t;
+    const ClassPairHost& cp = ctx->cps[i];
+    ClassWork w = work_of(ctx, cp, i);
+    o.mixed = mixed && cp.route ? 1 : 0;  // the launches of a build (run_classes)
+    if (o.mixed) {
+      hipLaunchKernelGGL(k_shift_tasks, dim3(grid_for(w.ntasks, 256)), dim3(256), 0, s, w.tasks, w.ntasks,
+                         (int)cp.unit_start, rt);
+      hipLaunchKernelGGL(k_route_tasks, dim3(grid_for(w.ntasks, 256)), dim3(256), 0, s, rt, w.ntasks, ctx->d_rpos,
+                         rt + tmax, rt + 2 * tmax);
+      HIP_CHECK(hipGetLastError());
+      w.units = ctx->d_units64;
+      w.tasks = rt + tmax;
+      w.units32 = ctx->d_units32;
+      w.tasks32 = rt + 2 * tmax;
+    }
     for (int r = 0; r <= reps; ++r) {
-      ClassWork w = work_of(ctx, ctx->cps[i], i);
       hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, w.queue, 1LL);
       hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, w.queue32, 1LL);
       HIP_CHECK(hipEventRecord(e0, s));
@@ -2252,15 +2287,19 @@ int asuka_jk_autotune(asuka_jk_ctx* ctx, const double* D, int flags, int reps, v
     if ((rc = time_class(i, &best))) return rc;
     if (eri_fast_has_plan(cp.la, cp.lb, cp.lc, cp.ld)) {
       // candidate shapes: 4 or 8 wavefronts per workgroup, 16..128 wave units
-      // per row task, LDS row accumulators on (where they fit) or off
+      // per row task (those that are different cuts), LDS row accumulators on
+      // (where they fit) or off
       int cC = 0, cD = 0;
       const bool fits = row_acc_fits(ctx, cp.la, cp.lb, cp.lc, cp.ld, &cC, &cD);
       int bw = cp.wpg, bt = cp.task_units;
       bool ba = cp.acc_colsC > 0;
       for (int acc = fits ? 1 : 0; acc >= 0; --acc)
-        for (int wpg : {4, 8})
+        for (int wpg : {4, 8}) {
+          int last = 0;  // the cut timed last (cut_units grows with tu)
           for (int tu : {16, 32, 64, 128}) {
             if ((rc = apply_shape(ctx, i, wpg, tu, acc != 0, s))) return rc;
+            if (cp.cut == last) continue;
+            last = cp.cut;
             double ms = 0.0;
             if ((rc = time_class(i, &ms))) return rc;
             if (ms < best) {
@@ -2270,6 +2309,7 @@ int asuka_jk_autotune(asuka_jk_ctx* ctx, const double* D, int flags, int reps, v
               ba = acc != 0;
             }
           }
+        }
       if ((rc = apply_shape(ctx, i, bw, bt, ba, s))) return rc;
     }
     cp.tuned_ms = std::max(best, 1e-6);

@@ -178,7 +178,6 @@ struct Chunk {
 // Wave votes through the ballot intrinsic, whose result the compiler knows to
 // be wave-uniform (branches on it stay scalar).
 __device__ __forceinline__ bool wave_any(bool v) { return __builtin_amdgcn_ballot_w64(v) != 0ull; }
-__device__ __forceinline__ bool wave_all(bool v) { return __builtin_amdgcn_ballot_w64(!v) == 0ull; }
 
 // A value known to be the same on every lane, moved to a scalar register.
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -221,9 +220,9 @@ struct FastArgs {
   const double *shell_xyz, *Q, *Dsp, *kq, *kd, *kcd;
   const int2 *kpp, *kao, *klao;
   FastDen den[2];
-  double eps_density, eps_prim, tau_mixed;
+  double eps_density, eps_prim;
   double ks;  // factor of the K sums: 1, or -1/2 for MODE_FOCK
-  int nden, ntasks, wpg, vote;  // vote: each kernel takes the units of its precision (mixed builds without routed lists)
+  int nden, ntasks, wpg;
   int acc_colsC, acc_colsD, lao_offC, lao_offD;
 };
 #define ASUKA_CONST __attribute__((address_space(4)))
@@ -739,11 +738,9 @@ __device__ __forceinline__ void dispatch_citem(int cc, ArgP ap, const Bra& br, i
 // J/K once at the end of the task.
 //
 // Precision: CT is the kernel's arithmetic. In mixed builds the FP64 and the
-// FP32 kernel each walk their own list of units (routed once per build);
-// without routed lists (vote) both walk all units, each from its own queue
-// head, and a unit goes to the FP32 kernel when every active quartet's bound
-// Q_ab Q_cd max|D| is below tau. Separate kernels keep the FP32 path's register
-// allocation (and so its occupancy) its own.
+// FP32 kernel of a split class pair each walk their own list of units, routed
+// once per build (k_route_units). Separate kernels keep the FP32 path's
+// register allocation (and so its occupancy) its own.
 // FX: accumulate in the 64-bit fixed point of deterministic builds
 // (EriOut::fixed), a separate instantiation so that the FP64-atomic kernels
 // carry none of its code or registers.
@@ -842,10 +839,6 @@ __global__ __launch_bounds__(kGroupThreads) void eri_fast_kernel(FastArgs args) 
                              fmax(cl(ap->Dsp, br.P), gl<double>(ap->kd + col, 8 * lane));
         if (ap->eps_density > 0.0) active = active && bound >= ap->eps_density;
         if (!wave_any(active)) continue;  // the whole unit is density-screened
-        if (ap->vote) {
-          const bool lowp = wave_all(!active || bound < ap->tau_mixed);
-          if (lowp != kF32) continue;  // the other precision's kernel takes this unit
-        }
         worked = true;
         // inactive lanes (tail, screened) run with an empty primitive loop and no
         // atomics so the wave stays converged for the cross-lane reductions
@@ -929,12 +922,12 @@ struct F32PlanOf {
   using type = Plan<PL::la, PL::lb, PL::lc, PL::ld, SA, SC>;
 };
 
-// The kernel arguments of a class pair's launch in one precision; false units
-// and tasks are w's (FP64 list) or, f32, the routed FP32 list.
+// The kernel arguments of a class pair's launch in one precision: f32 takes the
+// FP32 list of units and tasks (ClassWork::units32).
 inline FastArgs fast_args(const DevBasis& b, const ClassWork& w, const EriOut& o, bool f32) {
   FastArgs a{};
-  a.units = f32 && w.routed ? w.units32 : w.units;
-  a.tasks = f32 && w.routed ? w.tasks32 : w.tasks;
+  a.units = f32 ? w.units32 : w.units;
+  a.tasks = f32 ? w.tasks32 : w.tasks;
   a.queue = f32 ? w.queue32 : w.queue;
   a.pp = f32 ? (const void*)b.ppf32 : (const void*)b.ppf;
   a.kpd = f32 ? b.kp32d : b.kp64;
@@ -948,12 +941,11 @@ inline FastArgs fast_args(const DevBasis& b, const ClassWork& w, const EriOut& o
   const bool fock = o.mode == MODE_FOCK;
   a.den[0] = FastDen{o.D, fock ? o.F : o.J, fock ? o.F : o.K, o.Dpos, o.Jpos, o.Kc};
   a.den[1] = FastDen{o.D2, o.J2, o.K2, o.Dpos2, o.Jpos2, o.Kc2};
-  a.eps_density = o.eps_density, a.eps_prim = o.eps_prim, a.tau_mixed = o.tau_mixed;
+  a.eps_density = o.eps_density, a.eps_prim = o.eps_prim;
   a.ks = fock ? -0.5 : 1.0;
   a.nden = o.D2 ? 2 : 1;
   a.ntasks = (int)w.ntasks;
   a.wpg = w.wpg;
-  a.vote = o.mixed && !w.routed;
   a.acc_colsC = w.acc_colsC, a.acc_colsD = w.acc_colsD, a.lao_offC = w.lao_offC, a.lao_offD = w.lao_offD;
   return a;
 }

@@ -179,12 +179,10 @@ struct ClassWork {
   const int* q_cd;
   const long long* q_out_off;
   int cp_index;  // class-pair index (statistics counters)
-  // mixed builds with routed units (the vote taken once per build before the
-  // launches): the FP32 kernel's units and row tasks; units and tasks above
-  // then hold the FP64 kernel's. routed == 0: each kernel votes in place.
+  // split class pairs of mixed builds (EriOut::mixed): the FP32 kernel's units
+  // and row tasks; units and tasks above then hold the FP64 kernel's
   const WaveUnit* units32;
   const RowTask* tasks32;
-  int routed;
 };
 
 struct EriOut {
@@ -201,15 +199,15 @@ struct EriOut {
   // primitive quartets, [9] quartets evaluated in FP32, [10] their primitive quartets
   unsigned long long* counters;
   double eps_prim;    // primitive quartets with Q_p Q_q below this are skipped (0: none)
-  int mixed;          // allow the FP32 path
-  double tau_mixed;   // FP32 when Q_ab Q_cd max|D| < tau_mixed for the whole wave
+  int mixed;          // launch the FP32 kernel too, over ClassWork::units32
+  double tau_mixed;   // units go to FP32 when Q_ab Q_cd max|D| < tau_mixed for all of their quartets
   // MODE_JK with two densities (UHF/ROHF): each quartet is evaluated once and
   // digested with D into (J, K) and with D2 into (J2, K2); D2 == nullptr for one
   const double* D2;
   double* J2;
   double* K2;
-  // Ket-position buffers of the register kernels (null: J[c,d] by atomics on
-  // J and D[c,d] read from D). Ket lists (col_pair) are laid out in blocks of
+  // Ket-position buffers of the register kernels, which need them wherever J is
+  // wanted (the other kernels use J and D). Ket lists (col_pair) are laid out in blocks of
   // 64 positions of one ket class; block k holds component c (= ic * ND + id)
   // of the pair at position 64 k + lane at jblk[k] + 64 c + lane. A wave
   // unit starts at a block boundary, so its lanes read D[c,d] (Dpos, gathered

@@ -130,3 +130,28 @@ def test_graph_of_mixed_build_survives_retuning(gpu):
         torch.cuda.synchronize()
         for x, y, r in zip(out, eager, ref):
             assert float((x - r).abs().max()) < 1e-12 and float((y - r).abs().max()) < 1e-12
+
+
+def test_autotune_mixed_builds(gpu):
+    """Tuning for mixed builds runs each class pair as such a build does (one
+    FP64 launch, or the two routed ones) and leaves J and K what they were but
+    for the order of the sums (as above, 1e-12); tables that name the same cut
+    differently, and a fresh context under the table, likewise."""
+    from asuka_amd.hf.direct_jk import direct_JK
+
+    ao, ctx = _ctx(water_cluster(3, 5, "cc-pVDZ"), tau_mixed=1e-3)
+    C = np.linalg.qr(np.random.default_rng(7).standard_normal((ao.nao, 15)))[0]
+    D = 2.0 * C @ C.T
+    ref = direct_JK(ctx, D, mixed_precision=True)
+    ref64 = direct_JK(ctx, D, mixed_precision=False)
+    assert max(float((x - y).abs().max()) for x, y in zip(ref, ref64)) > 1e-11  # FP32 units among them
+    table = ctx.autotune(D, mixed_precision=True, reps=1)
+    assert all(t["tuned_ms"] > 0 for t in table)
+    _, fresh = _ctx(water_cluster(3, 5, "cc-pVDZ"), tau_mixed=1e-3)
+    fresh.set_tuning(table)
+    builds = [direct_JK(c, D, mixed_precision=True) for c in (ctx, fresh)]
+    for wpg, units in ((4, 1000), (8, 1000), (4, 2), (8, 2)):
+        ctx.set_tuning([dict(t, waves_per_group=wpg, units_per_task=units) for t in table])
+        builds.append(direct_JK(ctx, D, mixed_precision=True))
+    for got in builds:
+        assert all(float((x - y).abs().max()) < 1e-12 for x, y in zip(got, ref))
