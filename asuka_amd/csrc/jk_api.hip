@@ -495,8 +495,9 @@ __global__ void k_shift_tasks(const RowTask* __restrict__ tasks, long long ntask
 }
 
 // Counters (EriOut::counters) of a class pair of the register kernels, one
-// wavefront per wave unit: what those kernels evaluate follows from the
-// screening alone, so they carry no counting code. flags: the units' routing
+// wavefront per wave unit. Those kernels carry no counting code: this applies
+// their tests again, with the same bounds in the same arithmetic, so it says
+// what they are to evaluate, not what a launch did. flags: the units' routing
 // (k_route_units; null: all FP64).
 __global__ __launch_bounds__(256) void k_count_units(const DevBasis b, const WaveUnit* __restrict__ units,
                                                      long long nunits, const unsigned long long* __restrict__ flags,
@@ -505,6 +506,7 @@ __global__ __launch_bounds__(256) void k_count_units(const DevBasis b, const Wav
   const int lane = threadIdx.x & 63;
   for (long long k = blockIdx.x * 4LL + (threadIdx.x >> 6); k < nunits; k += gridDim.x * 4LL) {  // uniform per wave
     const WaveUnit un = units[k];
+    const bool f32 = flags && (flags[k] >> 32);
     const int P = un.P, pos = un.col + lane;
     bool active = lane < (int)un.ncol;
     if (active && eps_density > 0.0) active = (b.Q[P] * b.kq[pos]) * fmax(b.Dsp[P], b.kd[pos]) >= eps_density;
@@ -524,10 +526,15 @@ __global__ __launch_bounds__(256) void k_count_units(const DevBasis b, const Wav
     // and the lane slots the wave spends on them (64 x the longest lane)
     long long nev = 0;
     if (active && ur.ni > 0) {
-      const int cd0 = b.pp_start[Qp], ncd = min(b.pp_count[Qp], ur.j1);
-      const double kcut = eps_prim / b.ppf[b.pp_start[P]].q;  // the pair's largest, as the kernels
+      const int ab0 = b.pp_start[P], cd0 = b.pp_start[Qp], ncd = min(b.pp_count[Qp], ur.j1);
       int j = ur.j0;
-      while (j < ncd && !(b.ppf[cd0 + j].q < kcut)) ++j;
+      if (f32) {  // the cuts as run_chunk forms them
+        const float kcut = (float)(eps_prim * rcp_nr((double)b.ppf32[ab0].q));
+        while (j < ncd && !(b.ppf32[cd0 + j].q < kcut)) ++j;
+      } else {
+        const double kcut = eps_prim * rcp_nr(b.ppf[ab0].q);
+        while (j < ncd && !(b.ppf[cd0 + j].q < kcut)) ++j;
+      }
       nev = (long long)ur.ni * max(0, j - ur.j0);
     }
     const double nevs = wave_total((double)nev);
@@ -537,7 +544,7 @@ __global__ __launch_bounds__(256) void k_count_units(const DevBasis b, const Wav
       atomicAdd(cnt + 8, ksum);
       atomicAdd(cnt + 11, (unsigned long long)nevs);
       atomicAdd(cnt + 12, 64ull * (unsigned long long)nmax);
-      if (flags && (flags[k] >> 32)) {
+      if (f32) {
         atomicAdd(cnt + 9, nact);
         atomicAdd(cnt + 10, ksum);
       }

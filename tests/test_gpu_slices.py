@@ -45,7 +45,7 @@ def test_sliced_jk(gpu, oracle, ns, np_, nd, eps):
         J, K = direct_JK(ctx, D, stats=stats, **kw)
         tol = (1e-5 if kw.get("mixed_precision") else 1e-10) * scale
         assert np.abs(J.cpu().numpy() - Jr).max() < tol and np.abs(K.cpu().numpy() - Kr).max() < tol
-        # every quartet counted once, however many slices it has
+        # the counters take a quartet by its first slice alone
         assert stats["direct_jk_evaluated"] == ctx.ntasks
 
 
