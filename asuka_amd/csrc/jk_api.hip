@@ -812,6 +812,7 @@ static int pos_layout(asuka_jk_ctx* ctx, const std::vector<int>& col) {
       }
       kpoff[(size_t)k + 1] = kpoff[(size_t)k] + kmax;
     }
+    if (kpoff.back() * 64 >= (1LL << 31)) return fail(ASUKA_E_INVALID, "ket primitive-pair table exceeds 2^31 slots");
     const size_t nrow = (size_t)std::max<long long>(1, kpoff.back());
     std::vector<double> k64(nrow * 64 * kKet64, 0.0), k32d(nrow * 64 * kKet32d, 0.0);
     std::vector<float> k32f(nrow * 64 * kKet32f, 0.0f);
