@@ -80,3 +80,36 @@ def test_int1e_grad_against_differences(gpu, oracle, natm, spec):
     # one of the two matrices alone
     both = int1e_grad(ctx, Dh=Dh).cpu().numpy() + int1e_grad(ctx, Ws=Ws).cpu().numpy()
     assert np.abs(both - g).max() < 1e-11 * np.abs(g).max()
+
+
+def test_int1e_grad_beyond_the_lds_sums(gpu, oracle):
+    """513 nuclei, one more than the LDS sums of the nuclei's forces hold: they
+    go to the output one by one. Most are point charges without functions."""
+    from asuka_amd.hf.grad import int1e_grad
+
+    atoms = _atoms(3, 11)
+    ao, xyz, Z = _build(atoms, FULL)
+    rng = np.random.default_rng(12)
+    far = rng.uniform(-1.0, 1.0, size=(510, 3))
+    far *= (4.0 + 8.0 * rng.random((510, 1))) / np.linalg.norm(far, axis=1, keepdims=True)
+    Dh, Ws = (0.5 * (X + X.T) for X in rng.standard_normal((2, ao.nao, ao.nao)))
+    x0, Z = np.vstack([xyz, far]), np.concatenate([Z, np.full(510, 0.1)])
+    grads = [int1e_grad(_ctx(ao, x0[:n], Z[:n]), Dh=Dh, Ws=Ws).cpu().numpy() for n in (513, 512)]
+    assert np.abs(grads[0].sum(axis=0)).max() < 1e-10 * np.abs(grads[0]).max()
+    # the last charge on its own: what it adds to the others, and its force
+    Zl = np.where(np.arange(513) == 512, Z, 0.0)
+    last = int1e_grad(_ctx(ao, x0, Zl), Dh=Dh).cpu().numpy()
+    rest = int1e_grad(_ctx(ao, x0, 0.0 * Z), Dh=Dh).cpu().numpy()
+    diff = grads[0] - np.vstack([grads[1], np.zeros((1, 3))])
+    assert np.abs(diff - (last - rest)).max() < 1e-11 * np.abs(grads[0]).max()
+
+    def L(x):
+        S, T, V = oracle.int1e(_build([(s, p) for (s, _), p in zip(atoms, x)], FULL)[0], x, Z)
+        return float((Dh * (T + V)).sum() - (Ws * S).sum())
+
+    h = 5e-3
+    for k in (0, 7, 3 * 200 + 1, 3 * 512 + 2):
+        e = np.zeros((513, 3))
+        e.flat[k] = h
+        d = (8.0 * (L(x0 + e) - L(x0 - e)) - (L(x0 + 2 * e) - L(x0 - 2 * e))) / (12.0 * h)
+        assert abs(d - grads[0].flat[k]) < 1e-6 * np.abs(grads[0]).max(), k

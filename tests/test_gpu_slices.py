@@ -1,8 +1,11 @@
 """Wave units cut into slices of their primitive quartets (small contexts):
 contractions that leave only the bra, only the ket, both or neither to cut,
 counts around the cut sizes, with and without primitive screening, in J/K
-(FP64, mixed and reproducible) and in the derivative kernels, against the
-oracle. 1e-10 as in the other J/K tests: the slices only regroup sums."""
+(FP64, FP32, mixed and reproducible) and in the derivative kernels, against the
+oracle. 1e-10 as in the other J/K tests: the slices only regroup sums, and
+default mixed builds of contexts this small run all of it in FP64. With
+tau_mixed = 1e3 every quartet of the register kernels is FP32: roundings of 6e-8
+along chains of a few dozen operations, 2e-6."""
 
 import numpy as np
 import pytest
@@ -39,14 +42,19 @@ def test_sliced_jk(gpu, oracle, ns, np_, nd, eps):
     octx = oracle.make_context(ao)
     Jr, Kr = oracle.dense_JK(oracle.dense_eri(octx), D)
     ctx = make_direct_jk_context(ao, eps_schwarz=eps, eps_density=0.0)
+    ctx32 = make_direct_jk_context(ao, eps_schwarz=eps, eps_density=0.0, tau_mixed=1e3)
     scale = max(1.0, np.abs(Jr).max())
-    for kw in ({}, {"deterministic": True}, {"mixed_precision": True}):
+    for c, kw, tol in ((ctx, {"mixed_precision": False}, 1e-10), (ctx, {"deterministic": True}, 1e-10),
+                       (ctx, {"mixed_precision": True}, 1e-10), (ctx32, {"mixed_precision": True}, 2e-6)):
         stats = {}
-        J, K = direct_JK(ctx, D, stats=stats, **kw)
-        tol = (1e-5 if kw.get("mixed_precision") else 1e-10) * scale
-        assert np.abs(J.cpu().numpy() - Jr).max() < tol and np.abs(K.cpu().numpy() - Kr).max() < tol
+        J, K = direct_JK(c, D, stats=stats, **kw)
+        err = max(np.abs(J.cpu().numpy() - Jr).max(), np.abs(K.cpu().numpy() - Kr).max()) / scale
+        assert err < tol
         # the counters take a quartet by its first slice alone
-        assert stats["direct_jk_evaluated"] == ctx.ntasks
+        assert stats["direct_jk_evaluated"] == c.ntasks
+        for q in stats["class_counts"]:  # all FP32 or none, in the register kernels' classes
+            if q["prim_quartets_evaluated"]:
+                assert q["quartets_fp32"] == (q["bins"].sum() if c is ctx32 else 0)
 
 
 @pytest.mark.parametrize("ns,np_,nd", CASES)
@@ -69,8 +77,9 @@ def test_sliced_gradient(gpu, oracle, ns, np_, nd):
 def test_slices_skip_the_same_primitive_quartets(gpu):
     """A 4-water cluster alone (cut into slices) and beside a 12-water one in a
     batch (whose units are longer, so it is cut less) leave out the same
-    primitive quartets. The sums then differ by their order alone: about 4e4
-    terms into elements up to 1e2, under 2e-12 in the positions drawn here."""
+    primitive quartets in FP64. The sums then differ by their order alone: fewer
+    than 1e5 terms into elements below 1e2, whose roundings (1.4e-14 each at
+    most) add up as their square root, under 5e-12."""
     import torch
 
     from asuka_amd.basis import build_ao_basis_cart
@@ -83,8 +92,8 @@ def test_slices_skip_the_same_primitive_quartets(gpu):
         C, _ = np.linalg.qr(np.random.default_rng(2000 + seed).standard_normal((ao.nao, 5 * n)))
         aos.append(ao)
         Ds.append(torch.tensor(2.0 * C @ C.T, device="cuda"))
-    batch = direct_JK_batched(make_direct_jk_batch_context(aos, eps_schwarz=1e-12), Ds)
-    alone = direct_JK_batched([make_direct_jk_context(ao, eps_schwarz=1e-12) for ao in aos], Ds)
+    batch = direct_JK_batched(make_direct_jk_batch_context(aos, eps_schwarz=1e-12), Ds, mixed_precision=False)
+    alone = direct_JK_batched([make_direct_jk_context(ao, eps_schwarz=1e-12) for ao in aos], Ds, mixed_precision=False)
     for a, b in zip(batch, alone):
         for x, y in zip(a, b):
-            assert float((x - y).abs().max()) < 2e-12
+            assert float((x - y).abs().max()) < 2e-12  # well inside that
