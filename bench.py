@@ -61,8 +61,10 @@ def run_batched(args, cfg) -> int:
     water (seed 2000 + i), one batched J/K build per step on a batch context
     (one launch per class pair for the whole batch), eager and replayed from a
     captured HIP graph, with the default launch shapes and with the shapes the
-    autotuner picks on the largest molecule. The per-molecule-context path
-    (builds issued in turn) is timed beside it."""
+    autotuner picks on the largest molecule, in the package's default mixed
+    precision; the all-FP64 build is timed at the default shapes. The
+    per-molecule-context path (builds issued in turn) is timed beside it and its
+    J and K compared in both precisions."""
     import torch
 
     from asuka_amd.basis import build_ao_basis_cart
@@ -89,25 +91,28 @@ def run_batched(args, cfg) -> int:
     log(f"batch: {len(aos)} molecules, {sum(bc.naos)} AOs, {nq} Schwarz-screened quartets "
         f"(batch context {t_ctx:.1f}s, per-molecule contexts {t_ctxs:.1f}s)")
 
-    def measure(target):
-        out = direct_JK_batched(target, Ds)
+    def measure(target, mixed=True):
+        def run(out=None):
+            return direct_JK_batched(target, Ds, mixed_precision=mixed, out=out)
+
+        out = run()
         for _ in range(max(0, args.warmup)):
-            direct_JK_batched(target, Ds, out=out)
+            run(out)
         torch.cuda.synchronize(dev)
         t0 = time.perf_counter()
         for _ in range(args.steps):
-            direct_JK_batched(target, Ds, out=out)
+            run(out)
         torch.cuda.synchronize(dev)
         s_eager = (time.perf_counter() - t0) / args.steps
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(side):
-            direct_JK_batched(target, Ds, out=out)
+            run(out)
         torch.cuda.current_stream().wait_stream(side)
         torch.cuda.synchronize(dev)
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph):
-            direct_JK_batched(target, Ds, out=out)
+            run(out)
         graph.replay()
         torch.cuda.synchronize(dev)
         t0 = time.perf_counter()
@@ -116,20 +121,28 @@ def run_batched(args, cfg) -> int:
         torch.cuda.synchronize(dev)
         return s_eager, (time.perf_counter() - t0) / args.steps, [x.clone() for p in out for x in p if x is not None]
 
+    def diff(got, ref):
+        return max(float((a - b).abs().max()) for a, b in zip(got, ref))
+
     s_eager_m, s_graph_m, ref = measure(ctxs)
     log(f"per-molecule contexts: eager {s_eager_m * 1e3:.2f} ms, graph {s_graph_m * 1e3:.2f} ms")
     s_eager0, s_graph0, got0 = measure(bc)
-    d0 = max(float((a - b).abs().max()) for a, b in zip(got0, ref))
+    d0 = diff(got0, ref)
     log(f"batch context, default shapes: eager {s_eager0 * 1e3:.2f} ms, graph {s_graph0 * 1e3:.2f} ms "
         f"(max |dJ|,|dK| vs per-molecule contexts {d0:.1e})")
+    s_eager64, s_graph64, got64 = measure(bc, mixed=False)
+    ref64 = [x for p in direct_JK_batched(ctxs, Ds, mixed_precision=False) for x in p]
+    d64 = diff(got64, ref64)
+    log(f"batch context, FP64: eager {s_eager64 * 1e3:.2f} ms, graph {s_graph64 * 1e3:.2f} ms (max |dJ|,|dK| vs "
+        f"per-molecule contexts {d64:.1e}; mixed vs FP64 {diff(got0, got64):.1e})")
     # autotune on the largest molecule, apply its table to the batch
     big = int(np.argmax([a.nao for a in aos]))
     t0 = time.perf_counter()
-    table = ctxs[big].autotune(Ds[big])
+    table = ctxs[big].autotune(Ds[big], mixed_precision=True)
     bc.set_tuning(table)
     t_tune = time.perf_counter() - t0
     s_eager, s_graph, got = measure(bc)
-    dmax = max(float((a - b).abs().max()) for a, b in zip(got, ref))
+    dmax = diff(got, ref)
     log(f"batch context, autotuned shapes: eager {s_eager * 1e3:.2f} ms, graph {s_graph * 1e3:.2f} ms "
         f"(tuning {t_tune:.2f}s, max |dJ|,|dK| vs per-molecule contexts {dmax:.1e})")
     res = {
@@ -143,7 +156,7 @@ def run_batched(args, cfg) -> int:
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "f64",
+        "dtype": "f64+f32",
         "data": "synthetic (seeded water clusters, random orthonormal occupied orbitals)",
         "config": {"workload": cfg["workload"], "sizes": [int(n) for n in sizes], "basis": cfg["basis"],
                    "eps_schwarz": cfg["eps"], "launches": "one per class pair for the whole batch",
@@ -152,6 +165,8 @@ def run_batched(args, cfg) -> int:
         "s_per_batch_graph": s_graph,
         "graph_speedup": s_eager / s_graph,
         "default_shapes": {"s_per_batch_eager": s_eager0, "s_per_batch_graph": s_graph0},
+        "fp64": {"s_per_batch_eager": s_eager64, "s_per_batch_graph": s_graph64,
+                 "max_abs_dJK_vs_per_molecule_contexts": d64, "max_abs_dJK_mixed_vs_fp64": diff(got0, got64)},
         "autotuned_vs_default": s_graph0 / s_graph,
         "autotune_s": t_tune,
         "autotune_table_from": f"molecule {big} ({aos[big].nao} AOs), applied to the batch",
