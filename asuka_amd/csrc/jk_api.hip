@@ -53,8 +53,8 @@ static constexpr int kDefaultStreams = 4;
 static constexpr int kMaxStreams = 8;
 // LDS the register kernels of a class with nr roots hold for root tables
 static inline size_t root_table_lds(int nr) { return nr <= kLdsRootsMax ? rys_c::lds_table_bytes(nr) : 0; }
-// Accumulators up to this size run with 4-wave workgroups (16-unit tasks),
-// larger ones with 8-wave workgroups (32-unit tasks).
+// Accumulators up to this size run with 4-wave workgroups, larger ones with
+// 8-wave workgroups.
 static constexpr size_t kRowAccSmallBytes = 40 * 1024;
 // sqrt(2 pi^(5/2)), split evenly over the bra and ket primitive-pair factors
 static constexpr double kSqrt2Pi52 = 5.91496717279561287782;
@@ -120,9 +120,8 @@ struct ClassPairHost {
 // 32 % and 65 % slower than 48 for one water, and 2 %, 3 % and 4 % slower for
 // (H2O)7). Large contexts have no such unit and are left alone. Deterministic
 // builds run every unit whole (eri_fast_kernel). Measured with
-// kFillTasks: one water cc-pVDZ, mixed Fock build 2.37 -> 0.60 ms, (H2O)7 FP64
-// 4.66 -> 3.46 ms, (H2O)2 cc-pVTZ J/K 8.7 -> 3.8 ms, (H2O)5 two densities 3.68
-// -> 2.41 ms.
+// kFillTasks: one water cc-pVDZ, mixed Fock build 2.37 -> 0.66 ms, (H2O)7 FP64
+// 4.66 -> 3.64 ms, (H2O)5 two densities 3.68 -> 2.61 ms.
 static constexpr long long kSliceWaves = 8192;
 static inline long long slice_min(int nroots) { return std::max(2, 48 / (nroots * nroots)); }
 
@@ -241,7 +240,7 @@ static void slice_units(const std::vector<int>& blk_k, ClassPairHost& cp, const 
 // one wave item per wavefront, so that its units spread over the chip (1024
 // measured 1-4 % slower below 10 molecules: each task flushes its LDS sums).
 static constexpr long long kFillTasks = 512;
-static int cut_units(const ClassPairHost& cp, int task_units) {
+static int cut_units(const ClassPairHost& cp, int task_units) {  // units per task within these limits
   const int nit = std::max(1, eri_fast_nch(cp.la, cp.lb, cp.lc, cp.ld));
   return (int)std::min<long long>(
       task_units, std::max<long long>((cp.wpg + nit - 1) / nit, (cp.nunits + kFillTasks - 1) / kFillTasks));
@@ -759,7 +758,6 @@ static int route_task_layout(asuka_jk_ctx* ctx, hipStream_t s) {
   return ASUKA_OK;
 }
 
-// Device buffers of the routing of mixed builds (k_route_units and after).
 // Block offsets of the ket-position buffers (EriOut::jblk) for the padded ket
 // lists, and the buffers themselves.
 static int pos_layout(asuka_jk_ctx* ctx, const std::vector<int>& col) {
@@ -863,6 +861,7 @@ static int pos_layout(asuka_jk_ctx* ctx, const std::vector<int>& col) {
   return ASUKA_OK;
 }
 
+// Device buffers of the routing of mixed builds (k_route_units and after).
 static int route_alloc(asuka_jk_ctx* ctx, hipStream_t s) {
   bool any = false;
   for (const auto& cp : ctx->cps) any = any || cp.route;
