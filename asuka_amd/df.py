@@ -195,6 +195,12 @@ def cholesky_metric(V):
     raise RuntimeError("cholesky_metric failed after diagonal regularization retries")
 
 
+# Elements of a right-hand side that one triangular solve takes: beyond 128 MB
+# the library's workspace is refused (1145 x 15625, five waters in cc-pVDZ with
+# the default auxiliary set); 64 MB a solve.
+_SOLVE_ELEMENTS = 1 << 23
+
+
 def whiten_3c2e(X, L):
     """B = X L^-T (asuka/cueri/df.py:994): for X in the BQ layout (naux, nao, nao)
     B[Q] = sum_P (L^-1)_{QP} X[P], returned in the same layout."""
@@ -205,7 +211,13 @@ def whiten_3c2e(X, L):
         X2 = X.reshape(naux, -1)
     else:
         raise ValueError("X must be (naux, nao, nao) in the BQ layout")
-    B2 = torch.linalg.solve_triangular(L, X2, upper=False)
+    ncol = int(X2.shape[1])
+    step = max(1, _SOLVE_ELEMENTS // max(1, naux))
+    if ncol <= step:
+        return torch.linalg.solve_triangular(L, X2, upper=False).reshape(shape)
+    B2 = torch.empty_like(X2)
+    for k in range(0, ncol, step):
+        B2[:, k:k + step] = torch.linalg.solve_triangular(L, X2[:, k:k + step], upper=False)
     return B2.reshape(shape)
 
 

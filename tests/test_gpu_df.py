@@ -78,3 +78,31 @@ def test_df_jk_and_scf_against_oracle(gpu, oracle):
     # the DF energy is close to the exact (direct) one
     e_direct = run_hf_df(mol, two_e_backend="direct").scf.e_tot
     assert abs(res.scf.e_tot - e_direct) < 2e-3
+
+
+@pytest.mark.parametrize("naux,nao", [(1145, 125), (1374, 150), (3, 2000)])
+def test_whitening_in_several_solves(gpu, naux, nao):
+    """Right-hand sides beyond one solve's share (the last part ragged): L B = X
+    to rounding, and the first columns as one solve gives them."""
+    from asuka_amd.df import whiten_3c2e
+
+    torch = gpu
+    g = torch.Generator(device="cuda").manual_seed(naux)
+    A = torch.randn(naux, naux, dtype=torch.float64, device="cuda", generator=g)
+    L = torch.linalg.cholesky(A @ A.T / naux + torch.eye(naux, dtype=torch.float64, device="cuda"))
+    X = torch.randn(naux, nao, nao, dtype=torch.float64, device="cuda", generator=g)
+    B = whiten_3c2e(X, L)
+    assert B.shape == X.shape
+    assert float((L @ B.reshape(naux, -1) - X.reshape(naux, -1)).abs().max()) < 1e-12
+    one = torch.linalg.solve_triangular(L, X[:, 0, :].contiguous(), upper=False)
+    assert float((B[:, 0, :] - one).abs().max()) < 1e-12
+
+
+def test_df_scf_of_five_waters(gpu):
+    """The default backend beyond one solve's share, near the direct energy."""
+    from asuka_amd.frontend import run_hf_df
+
+    mol = water_cluster(5, 3, "cc-pVDZ")
+    df = run_hf_df(mol, two_e_backend="df").scf
+    direct = run_hf_df(mol, two_e_backend="direct").scf
+    assert df.converged and abs(df.e_tot - direct.e_tot) < 5 * 2e-3
